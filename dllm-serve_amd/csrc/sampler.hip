@@ -86,19 +86,17 @@ __device__ __forceinline__ float gumbel_value(float l, double T, uint64_t seed, 
 // Fold 8 logits (one 16-byte chunk starting at column e0) into the running
 // (m, s, i).  A thread's chunks arrive in increasing column order, so a tie
 // with the running max keeps the earlier index.
-template <bool GUMBEL>
-__device__ __forceinline__ void smx_chunk(u32x4_t v, int e0, float& m, float& s, int& i, double T = 0.0,
-                                          uint64_t seed = 0, uint64_t c0 = 0) {
-  float f[8];
+__device__ __forceinline__ void smx_unpack(u32x4_t v, float (&f)[8]) {
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
     f[2 * w] = __uint_as_float(v[w] << 16);
     f[2 * w + 1] = __uint_as_float(v[w] & 0xffff0000u);
   }
-  if (GUMBEL) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) f[k] = gumbel_value(f[k], T, seed, c0 + (uint64_t)k);
-  }
+}
+
+__device__ __forceinline__ void smx_chunk(u32x4_t v, int e0, float& m, float& s, int& i) {
+  float f[8];
+  smx_unpack(v, f);
   const float cm = fmaxf(fmaxf(fmaxf(f[0], f[1]), fmaxf(f[2], f[3])), fmaxf(fmaxf(f[4], f[5]), fmaxf(f[6], f[7])));
   if (cm > m) {
     int k = 7;
@@ -114,6 +112,99 @@ __device__ __forceinline__ void smx_chunk(u32x4_t v, int e0, float& m, float& s,
 #pragma unroll
     for (int k = 0; k < 8; ++k) e[k] = fexp2((f[k] - m) * kLog2e);
     s += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+  }
+}
+
+// The noisy rows.  v = exp(l) / E^T, E = -log u, takes ~160 instructions of
+// f64 per logit, but next to the row's maximum only few values count: one that
+// lies kNoiseGap below any other value of the row adds exp(-kNoiseGap) < 2^-158
+// of that value's own term to the sum of exponentials -- nothing in f32 -- and
+// is not the maximum.  A cheap bound tells most of them: with h = the high 32
+// bits of the draw, E >= 1 - u > (2^32 - 1 - h) 2^-32, hence
+//   log2 v < l log2(e) - T (log2(2^32 - 1 - h) - 32).
+// The wavefront keeps a threshold from the largest value any of its lanes has
+// computed; a logit whose bound is below it is left out, all others (infinite
+// and NaN bounds included) are computed in f64 as before.  Per chunk the lanes
+// first compute the candidate with their largest bound, so that already the
+// first chunk of a row leaves one or two f64 evaluations for 512 logits.
+// Bounded by the integer hash (two 64-bit products per logit).
+// 256 x 126464 logits at temperature 1 on an MI355X: 154 -> 42 us.
+constexpr float kNoiseGap = 110.0f;
+
+// log2 of the bound above for one logit; z1 = seed + (counter + 1) * golden.
+__device__ __forceinline__ float noise_bound_log2(float l, float T, uint64_t z1) {
+  uint64_t z = z1;
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z ^= z >> 27;
+  const uint32_t lo = (uint32_t)z, hi = (uint32_t)(z >> 32);
+  // high word of z * 0x94D049BB133111EB, then of its xor with itself >> 31
+  uint32_t h = __umulhi(lo, 0x133111EBu) + lo * 0x94D049BBu + hi * 0x133111EBu;
+  h ^= h >> 31;
+  const float lg = __builtin_amdgcn_logf((float)~h) - 32.0f;  // log2; -inf when ~h is 0
+  return __builtin_fmaf(l, kLog2e, -T * lg);
+}
+
+// log2 below which a bound means "kNoiseGap below m_w, or less" (m_w: a value
+// of the row).  The slack covers the bound's f32 rounding (log2 terms below
+// 2^9, T times one of at most 32) and the rounding of v to bf16 (2^-8); up to
+// 2^127 only, so that every value that may overflow is computed.
+__device__ __forceinline__ float noise_threshold(float m_w, float T) {
+  const float d = m_w - kNoiseGap;
+  return d > 1.0f ? fminf(__builtin_amdgcn_logf(d), 127.0f) - (0.02f + 1e-4f * T) : -INFINITY;
+}
+
+__device__ __forceinline__ float wave_max(float x) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) x = fmaxf(x, __uint_as_float(lane_xor(__float_as_uint(x), off)));
+  return x;
+}
+
+// Fold 8 logits of a row with temperature T into (m, s, i); rc + e0 = counter
+// of the first.  thr: the wavefront's threshold.  All 64 lanes call it; those
+// with `live` false hold no logits.
+__device__ __forceinline__ void smx_noisy_chunk(u32x4_t v, int e0, bool live, double T, uint64_t seed, uint64_t rc,
+                                                float& m, float& s, int& i, float& thr) {
+  float f[8], b[8];
+  smx_unpack(v, f);
+  const float Tf = (float)T;
+  uint64_t z = seed + (rc + (uint64_t)e0 + 1) * 0x9E3779B97F4A7C15ull;
+  uint32_t pend = 0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    b[k] = noise_bound_log2(f[k], Tf, z);
+    z += 0x9E3779B97F4A7C15ull;
+    pend |= !(b[k] < thr) ? 1u << k : 0u;
+  }
+  if (!live) pend = 0;
+  while (__builtin_amdgcn_ballot_w64(pend != 0)) {  // each turn clears one bit of every lane that has any
+    bool raised = false;
+    if (pend != 0) {
+      int at = -1;
+      float bb = 0.f, l = 0.f;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const bool take = ((pend >> k) & 1u) && (at < 0 || !(b[k] <= bb));
+        at = take ? k : at;
+        bb = take ? b[k] : bb;
+        l = take ? f[k] : l;
+      }
+      pend &= ~(1u << at);
+      const float x = gumbel_value(l, T, seed, rc + (uint64_t)(e0 + at));
+      if (x > m) {
+        s = s * fexp2((m - x) * kLog2e) + fexp2((x - x) * kLog2e);
+        m = x;
+        i = e0 + at;
+        raised = true;
+      } else if (m != -INFINITY) {
+        s += fexp2((x - m) * kLog2e);
+        if (x == m) i = min(i, e0 + at);
+      }
+    }
+    if (__builtin_amdgcn_ballot_w64(raised)) {
+      thr = fmaxf(thr, noise_threshold(wave_max(m), Tf));
+#pragma unroll
+      for (int k = 0; k < 8; ++k) pend &= b[k] < thr ? ~(1u << k) : ~0u;
+    }
   }
 }
 
@@ -138,7 +229,10 @@ __device__ __forceinline__ void smx_scan(const SmxArgs& a, int row, int c0, int 
   const u32x4_t ninf = {0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
   const double T = GUMBEL ? a.temp[row] : 0.0;
   const uint64_t rc = GUMBEL ? (uint64_t)(a.row_base + row) * (uint64_t)a.V : 0;
-  for (int c = c0 + (int)threadIdx.x; c < c1; c += 4 * NT) {
+  float thr = -INFINITY;
+  // noisy rows: whole wavefronts walk together (their lanes share a threshold)
+  const int lead = GUMBEL && T > 0.0 ? (int)(threadIdx.x & 63) : 0;
+  for (int c = c0 + (int)threadIdx.x; c - lead < c1; c += 4 * NT) {
     u32x4_t v[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -148,10 +242,10 @@ __device__ __forceinline__ void smx_scan(const SmxArgs& a, int row, int c0, int 
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int e0 = 8 * (c + u * NT);
-      if (GUMBEL && T > 0.0 && c + u * NT < c1)  // padding chunks stay -inf
-        smx_chunk<true>(v[u], e0, m, s, idx, T, a.seed, rc + (uint64_t)e0);
+      if (GUMBEL && T > 0.0)
+        smx_noisy_chunk(v[u], e0, c + u * NT < c1, T, a.seed, rc, m, s, idx, thr);
       else
-        smx_chunk<false>(v[u], e0, m, s, idx);
+        smx_chunk(v[u], e0, m, s, idx);
     }
   }
 }

@@ -251,3 +251,33 @@ def test_remask_sampler_with_temperature(dev):
     got = tok.cpu().numpy().reshape(-1)
     assert np.mean(got == want) > 0.99   # rows whose f64 noise rounds differently may pick another token
     assert np.array_equal(got != MASK, want != MASK) or np.mean((got != MASK) == (want != MASK)) > 0.99
+
+
+@pytest.mark.parametrize("M,V,sigma,T", [
+    (3, 8, 1.0, 1.0),            # one chunk: lanes without logits
+    (5, 520, 0.1, 1.0),          # 65 chunks, small values: nothing may be left out
+    (9, 1032, 2.0, 0.25),
+    (513, 4104, 3.0, 0.7),       # 256-thread workgroups
+    (4, 33288, 6.0, 3.0),        # a second round of loads, partly past the row's end
+])
+def test_softmax_max_sample_bounds(dev, M, V, sigma, T):
+    """The bound that leaves logits out of the f64 transform: row lengths at
+    the edges of the chunk walk, values below and far above the gap."""
+    print(f"softmax_max_sample bounds M={M} V={V} sigma={sigma} T={T}", flush=True)
+    g = torch.Generator().manual_seed(M + V)
+    t = (torch.randn(M, V, generator=g) * sigma).to(torch.bfloat16)
+    t[0, ::3] = -float("inf")
+    x0, p = _run_k8_sample(t.to(dev), [T] * M, 99, 5)
+    _check_sample(bits(t), np.full(M, T), 99, 5, x0, p)
+
+
+def test_softmax_max_sample_overflow(dev):
+    """Values past the largest bf16 are infinite (the reference's too): the
+    first infinite one is the token, its probability NaN."""
+    print("softmax_max_sample overflow", flush=True)
+    t = torch.zeros(2, 8200, dtype=torch.bfloat16)
+    t[0, [700, 41, 8199]] = 95.0     # exp(95) / E > 3.4e38 for every draw (E < 37)
+    t[1, [8199, 3000]] = 80.0        # large, finite
+    x0, p = _run_k8_sample(t.to(dev), [1.0, 1.0], 7, 0)
+    assert x0[0] == 41 and np.isnan(torch.from_numpy(p[:1].view(np.int16)).view(torch.bfloat16).float().item())
+    _check_sample(bits(t[1:]), np.array([1.0]), 7, 1, x0[1:], p[1:])

@@ -101,7 +101,9 @@ def _unmask_case(rng, n_seq, max_win, tie_levels):
     return np.array(tokens, np.int64), params, conf, x0
 
 
-@pytest.mark.parametrize("n_seq,max_win,ties", [(64, 300, 0), (64, 300, 16), (8, 8192, 64), (3, 1, 0), (32, 64, 2)])
+@pytest.mark.parametrize("n_seq,max_win,ties", [(64, 300, 0), (64, 300, 16), (8, 8192, 64), (3, 1, 0), (32, 64, 2),
+                                               (20, 65, 4), (20, 256, 0), (20, 257, 3), (20, 1024, 8),
+                                               (20, 1025, 8)])  # edges of the one-wavefront forms
 def test_unmask_matches_oracle(dev, n_seq, max_win, ties):
     print(f"unmask n_seq={n_seq} max_win={max_win} ties={ties}", flush=True)
     rng = np.random.default_rng(n_seq * 31 + max_win + ties)

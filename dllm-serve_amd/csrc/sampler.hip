@@ -12,11 +12,12 @@
 // |m| <= 2, in which case the columns before that index are rescanned for an
 // earlier one whose rounded probability ties.
 //
-// Layout: one workgroup per row (1024 threads when there are at most 512
-// rows, else 256); each thread streams every NT-th 16-byte chunk with four
-// loads in flight and keeps a record {m, s, first index of m}; the records
-// are merged across the workgroup and one wavefront finishes the row (the
-// tie rescan included).  HBM-bound: 2 V bytes per row, read once.
+// Layout: one workgroup per row, or several for few rows (smx_splits); each
+// thread streams every NT-th 16-byte chunk, the next batch's loads in flight,
+// and keeps a record {m, s, first index of m}; the records are merged across
+// the workgroup (and across a row's workgroups by a second launch) and one
+// wavefront finishes the row (the tie rescan included).  HBM-bound: 2 V bytes
+// per row, read once.  256 rows of 126464: 16.4 -> 14.3 us (4.5 TB/s).
 //
 // With a per-row temperature T > 0 the row is first transformed as the
 // reference's add_gumbel_noise does (model_runner.py:592-600):
@@ -84,9 +85,6 @@ __device__ __forceinline__ float gumbel_value(float l, double T, uint64_t seed, 
   return bf16_bits_to_f32(f64_to_bf16_bits_2step(v));
 }
 
-// Fold 8 logits (one 16-byte chunk starting at column e0) into the running
-// (m, s, i).  A thread's chunks arrive in increasing column order, so a tie
-// with the running max keeps the earlier index.
 __device__ __forceinline__ void smx_unpack(u32x4_t v, float (&f)[8]) {
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
@@ -95,24 +93,41 @@ __device__ __forceinline__ void smx_unpack(u32x4_t v, float (&f)[8]) {
   }
 }
 
-__device__ __forceinline__ void smx_chunk(u32x4_t v, int e0, float& m, float& s, int& i) {
-  float f[8];
-  smx_unpack(v, f);
-  const float cm = fmaxf(fmaxf(fmaxf(f[0], f[1]), fmaxf(f[2], f[3])), fmaxf(fmaxf(f[4], f[5]), fmaxf(f[6], f[7])));
-  if (cm > m) {
-    int k = 7;
+// Fold U chunks of 8 logits (chunk u = columns 8 (c + u step) ..) into the
+// running (m, s, i).  A thread's chunks arrive in increasing column order, so
+// a tie with the running max keeps the earlier index.  One test of the maximum
+// for all 8 U logits.
+template <int U>
+__device__ __forceinline__ void smx_batch(const u32x4_t (&v)[U], int c, int step, float& m, float& s, int& i) {
+  float f[U][8];
 #pragma unroll
-    for (int kk = 6; kk >= 0; --kk)
-      if (f[kk] == cm) k = kk;
+  for (int u = 0; u < U; ++u) smx_unpack(v[u], f[u]);
+  float cm = f[0][0];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int k = 0; k < 8; ++k) cm = fmaxf(cm, f[u][k]);
+  if (cm > m) {
+    int at = 0;
+#pragma unroll
+    for (int u = U - 1; u >= 0; --u)
+#pragma unroll
+      for (int k = 7; k >= 0; --k)
+        if (f[u][k] == cm) at = 8 * (c + u * step) + k;
     s *= fexp2((m - cm) * kLog2e);
     m = cm;
-    i = e0 + k;
+    i = at;
   }
   if (m != -INFINITY) {
-    float e[8];
+    float e0 = 0.f, e1 = 0.f;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) e[k] = fexp2((f[k] - m) * kLog2e);
-    s += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int k = 0; k < 8; k += 2) {
+        e0 += fexp2((f[u][k] - m) * kLog2e);
+        e1 += fexp2((f[u][k + 1] - m) * kLog2e);
+      }
+    s += e0 + e1;
   }
 }
 
@@ -220,19 +235,51 @@ struct SmxArgs {
   const double* temp;  // per-row temperature (nullable: no transform)
   uint64_t seed;
   int64_t row_base;
+  int n_split;         // workgroups per row
+  float* rec;          // [M][n_split][3] records (n_split > 1)
 };
 
 // Fold columns [8 c0, 8 c1) of one row into the thread's running (m, s, i):
-// thread t takes chunks c0 + t, c0 + t + NT, ..., four 16-byte loads in flight.
-template <bool GUMBEL, int NT>
+// thread t takes chunks c0 + t, c0 + t + NT, ..., four 16-byte loads of the
+// next batch in flight beside the batch that is summed.
+template <int NT>
 __device__ __forceinline__ void smx_scan(const SmxArgs& a, int row, int c0, int c1, float& m, float& s, int& idx) {
+  constexpr int U = 4;
   const uint16_t* base = a.logits + (int64_t)row * a.ld;
   const u32x4_t ninf = {0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
-  const double T = GUMBEL ? a.temp[row] : 0.0;
-  const uint64_t rc = GUMBEL ? (uint64_t)(a.row_base + row) * (uint64_t)a.V : 0;
+  const int nb = (c1 - c0 + U * NT - 1) / (U * NT);
+  if (nb <= 0) return;
+  int c = c0 + (int)threadIdx.x;
+  u32x4_t v[U];
+  // chunks past the end re-read the last one and are replaced by -inf below
+#pragma unroll
+  for (int u = 0; u < U; ++u) v[u] = ld128_stream(base + 8 * (int64_t)min(c + u * NT, c1 - 1));
+  for (int b = 1; b < nb; ++b) {
+    u32x4_t w[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) w[u] = ld128_stream(base + 8 * (int64_t)min(c + (U + u) * NT, c1 - 1));
+    smx_batch<U>(v, c, NT, m, s, idx);
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = w[u];
+    c += U * NT;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (c + u * NT >= c1) v[u] = ninf;
+  smx_batch<U>(v, c, NT, m, s, idx);
+}
+
+// The same for a row with temperature T > 0 (smx_noisy_chunk).  Whole
+// wavefronts walk together: their lanes share a threshold.
+template <int NT>
+__device__ __forceinline__ void smx_scan_noisy(const SmxArgs& a, int row, int c0, int c1, float& m, float& s,
+                                               int& idx) {
+  const uint16_t* base = a.logits + (int64_t)row * a.ld;
+  const u32x4_t ninf = {0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
+  const double T = a.temp[row];
+  const uint64_t rc = (uint64_t)(a.row_base + row) * (uint64_t)a.V;
   float thr = -INFINITY;
-  // noisy rows: whole wavefronts walk together (their lanes share a threshold)
-  const int lead = GUMBEL && T > 0.0 ? (int)(threadIdx.x & 63) : 0;
+  const int lead = (int)(threadIdx.x & 63);
   for (int c = c0 + (int)threadIdx.x; c - lead < c1; c += 4 * NT) {
     u32x4_t v[4];
 #pragma unroll
@@ -241,13 +288,8 @@ __device__ __forceinline__ void smx_scan(const SmxArgs& a, int row, int c0, int 
       v[u] = cc < c1 ? ld128_stream(base + 8 * (int64_t)cc) : ninf;
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int e0 = 8 * (c + u * NT);
-      if (GUMBEL && T > 0.0)
-        smx_noisy_chunk(v[u], e0, c + u * NT < c1, T, a.seed, rc, m, s, idx, thr);
-      else
-        smx_chunk(v[u], e0, m, s, idx);
-    }
+    for (int u = 0; u < 4; ++u)
+      smx_noisy_chunk(v[u], 8 * (c + u * NT), c + u * NT < c1, T, a.seed, rc, m, s, idx, thr);
   }
 }
 
@@ -317,15 +359,66 @@ __device__ void smx_finish(const SmxArgs& a, int row, float m, float s, int idx)
   }
 }
 
-// One workgroup per row: scan, merge and finish in one launch.
+// One workgroup per row (n_split = 1: scan, merge and finish in one launch) or
+// n_split of them, each a range of the row's chunks; their records (m, s, i)
+// then go to `rec` and smx_merge_kernel finishes the rows.
 template <bool GUMBEL, int NT>
 __global__ __launch_bounds__(NT) void smx_row_kernel(SmxArgs a) {
-  const int row = blockIdx.x;
+  const int row = blockIdx.x / a.n_split;
+  const int sp = blockIdx.x - row * a.n_split;
+  const int per = (a.chunks + a.n_split - 1) / a.n_split;
+  const int c0 = sp * per, c1 = min(a.chunks, c0 + per);
   float m = -INFINITY, s = 0.f;
   int idx = INT_MAX;
-  smx_scan<GUMBEL, NT>(a, row, 0, a.chunks, m, s, idx);
+  if (GUMBEL && a.temp[row] > 0.0)
+    smx_scan_noisy<NT>(a, row, c0, c1, m, s, idx);
+  else
+    smx_scan<NT>(a, row, c0, c1, m, s, idx);
   smx_block_reduce<NT>(m, s, idx);
-  if ((threadIdx.x >> 6) == 0) smx_finish(a, row, m, s, idx);
+  if (a.n_split > 1) {
+    if (threadIdx.x == 0) {
+      float* r = a.rec + 3 * (int64_t)blockIdx.x;
+      r[0] = m;
+      r[1] = s;
+      r[2] = __int_as_float(idx);
+    }
+  } else if ((threadIdx.x >> 6) == 0) {
+    smx_finish(a, row, m, s, idx);
+  }
+}
+
+// The records of a row's n_split (at most 64) ranges merged, one wavefront per row.
+__global__ __launch_bounds__(256) void smx_merge_kernel(SmxArgs a) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (row >= a.M) return;
+  float m = -INFINITY, s = 0.f;
+  int idx = INT_MAX;
+  if (lane < a.n_split) {
+    const float* r = a.rec + 3 * ((int64_t)row * a.n_split + lane);
+    m = r[0];
+    s = r[1];
+    idx = __float_as_int(r[2]);
+  }
+  smx_wave_reduce(m, s, idx);
+  smx_finish(a, row, m, s, idx);
+}
+
+// Workgroups per row.  A CU takes in at most ~26 GB a millisecond, ~10 us for a
+// row of 253 KB, so few rows are spread over several CUs; the second launch
+// (~2.5 us) pays for that up to 64 rows, and with noise, whose integer hash
+// keeps a CU busy for 40 us a row, wherever CUs would stay idle.  Measured at
+// 126464 logits per row, one workgroup a row against the split: 8 rows 12.3 /
+// 7.8, 32 12.5 / 8.5, 64 12.3 / 9.8, 96 12.4 / 11.6, 128 12.6 / 12.1 us (not
+// split); with noise 8 rows 42 / 17.5, 64 42 / 21.8, 128 42 / 30.5 us.  A range
+// is at least one chunk per thread.
+static int smx_splits(int M, int V, bool noisy) {
+  if (M <= 0 || M > (noisy ? 128 : 64)) return 1;
+  int n = 256 / M;
+  if (n > 8) n = 8;
+  const int most = V / 8 / (noisy ? 1024 : 512);
+  if (n > most) n = most;
+  return n < 1 ? 1 : n;
 }
 
 // ---- K9 ---------------------------------------------------------------------
@@ -482,12 +575,18 @@ using namespace dllm;
 extern "C" size_t dllm_softmax_max_workspace_size(int M, int V) {
   (void)M;
   (void)V;
-  return 0;  // one workgroup per row: no partial records
+  return 0;  // nothing is required
+}
+
+extern "C" size_t dllm_softmax_max_split_workspace_size(int M, int V) {
+  // the noisy form's ranges are the most
+  const int n = M > 0 && V > 0 ? max(smx_splits(M, V, true), smx_splits(M, V, false)) : 1;
+  return n > 1 ? (size_t)M * n * 3 * sizeof(float) : 0;
 }
 
 static int softmax_max_launch(const char* name, const uint16_t* logits, int64_t ld, int M, int V,
                               const double* row_temperature, uint64_t seed, int64_t row_base, int64_t* x0,
-                              uint16_t* x0_p, void* stream) {
+                              uint16_t* x0_p, void* workspace, size_t workspace_bytes, void* stream) {
   if (M < 0 || V < 0) return fail(DLLM_ERR_INVALID_ARG, "%s: negative size", name);
   if (M == 0) return DLLM_OK;
   if (V == 0 || V % 8 != 0)
@@ -508,37 +607,48 @@ static int softmax_max_launch(const char* name, const uint16_t* logits, int64_t 
   a.seed = seed;
   a.row_base = row_base;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)M);
-  // few rows: 1024 threads per row keep enough loads in flight per CU
-  if (M <= 512) {
-    if (row_temperature)
+  // without a workspace that holds the records every row is one workgroup's
+  a.n_split = smx_splits(M, V, row_temperature != nullptr);
+  a.rec = reinterpret_cast<float*>(workspace);
+  if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 4 ||
+      workspace_bytes < (size_t)M * a.n_split * 3 * sizeof(float) || (int64_t)M * a.n_split > INT32_MAX)
+    a.n_split = 1;
+  const dim3 grid((unsigned)(M * a.n_split));
+  // Threads per row.  Measured in us, 1024 / 512 / 256 threads: 8 rows 13.3 /
+  // 13.1 / 16.4, 256 rows 17.1 / 15.1 / 17.1, 384 rows 28.7 / 24.7 / 23.4, 1024
+  // rows 59.2 / 47.0 / 45.8.  Noisy rows are bound by the hash: as many
+  // wavefronts as the rows leave room for.
+  if (row_temperature) {
+    if (M <= 512)
       smx_row_kernel<true, 1024><<<grid, dim3(1024), 0, st>>>(a);
     else
-      smx_row_kernel<false, 1024><<<grid, dim3(1024), 0, st>>>(a);
-  } else {
-    if (row_temperature)
       smx_row_kernel<true, 256><<<grid, dim3(256), 0, st>>>(a);
+  } else {
+    if (M <= 256)
+      smx_row_kernel<false, 512><<<grid, dim3(512), 0, st>>>(a);
     else
       smx_row_kernel<false, 256><<<grid, dim3(256), 0, st>>>(a);
   }
-  return check_launch(name);
+  int rc = check_launch(name);
+  if (rc == DLLM_OK && a.n_split > 1) {
+    smx_merge_kernel<<<dim3((unsigned)((M + 3) / 4)), dim3(256), 0, st>>>(a);
+    rc = check_launch(name);
+  }
+  return rc;
 }
 
 extern "C" int dllm_softmax_max(const uint16_t* logits, int64_t ld, int M, int V, int64_t* x0, uint16_t* x0_p,
                                 void* workspace, size_t workspace_bytes, void* stream) {
-  (void)workspace;
-  (void)workspace_bytes;
-  return softmax_max_launch("dllm_softmax_max", logits, ld, M, V, nullptr, 0, 0, x0, x0_p, stream);
+  return softmax_max_launch("dllm_softmax_max", logits, ld, M, V, nullptr, 0, 0, x0, x0_p, workspace, workspace_bytes,
+                            stream);
 }
 
 extern "C" int dllm_softmax_max_sample(const uint16_t* logits, int64_t ld, int M, int V,
                                        const double* row_temperature, uint64_t seed, int64_t row_base, int64_t* x0,
                                        uint16_t* x0_p, void* workspace, size_t workspace_bytes, void* stream) {
   if (row_base < 0) return fail(DLLM_ERR_INVALID_ARG, "dllm_softmax_max_sample: negative row_base");
-  (void)workspace;
-  (void)workspace_bytes;
   return softmax_max_launch("dllm_softmax_max_sample", logits, ld, M, V, row_temperature, seed, row_base, x0, x0_p,
-                            stream);
+                            workspace, workspace_bytes, stream);
 }
 
 extern "C" int dllm_lowconf_unmask(int64_t* tokens, int64_t n_tokens, const int32_t* seq_params, int n_seq,

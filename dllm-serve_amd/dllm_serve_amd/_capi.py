@@ -66,6 +66,7 @@ SIGNATURES = {
     ),
     "dllm_rope_neox": (_I, [_P, _I64, _P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _I, _I, _I, _I, _P]),
     "dllm_softmax_max_workspace_size": (_SZ, [_I, _I]),
+    "dllm_softmax_max_split_workspace_size": (_SZ, [_I, _I]),
     "dllm_softmax_max": (_I, [_P, _I64, _I, _I, _P, _P, _P, _SZ, _P]),
     "dllm_softmax_max_sample": (_I, [_P, _I64, _I, _I, _P, ctypes.c_uint64, _I64, _P, _P, _P, _SZ, _P]),
     "dllm_lowconf_unmask": (_I, [_P, _I64, _P, _I, _I, _P, _P, _I64, _I64, _P, _P]),
@@ -343,9 +344,15 @@ def softmax_max_workspace_size(M, V) -> int:
     return int(load().dllm_softmax_max_workspace_size(M, V))
 
 
+def softmax_max_split_workspace_size(M, V) -> int:
+    """Bytes with which softmax_max spreads few rows over several workgroups (0: it would not)."""
+    return int(_lib_now().dllm_softmax_max_split_workspace_size(M, V))
+
+
 def softmax_max(logits, x0, x0_p, workspace=None):
     """K8: x0_p, x0 = max(softmax(logits, -1), -1) of bf16 logits [M, V]
-    (x0 int64 [M], x0_p bf16 [M]).  workspace is optional (the kernel needs none)."""
+    (x0 int64 [M], x0_p bf16 [M]).  workspace is optional
+    (see softmax_max_split_workspace_size)."""
     _require_gpu(logits, x0, x0_p, workspace)
     lib = load()
     M, V = logits.shape

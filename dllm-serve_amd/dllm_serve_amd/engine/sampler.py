@@ -82,15 +82,11 @@ class RemaskSampler:
         self.max_logprobs = max_logprobs  # rows per LM-head chunk (None: all at once)
         self.seed = int(seed)             # base of the per-call noise seeds (temperature > 0)
         self.calls = 0
-        self._ws = None
 
     def _workspace(self, M: int, V: int, device) -> Optional[torch.Tensor]:
-        need = _capi.softmax_max_workspace_size(M, V)
-        if need == 0:
-            return None
-        if self._ws is None or self._ws.numel() < need or self._ws.device != device:
-            self._ws = torch.empty(max(need, 16), dtype=torch.uint8, device=device)
-        return self._ws
+        # from the allocator at every call: a sampler may be used on several streams
+        need = _capi.softmax_max_split_workspace_size(M, V)
+        return torch.empty(need, dtype=torch.uint8, device=device) if need else None
 
     def logits_max(self, rows: torch.Tensor, row_temperature: Optional[torch.Tensor] = None, seed: int = 0):
         """x0 (int64) and x0_p (bf16) of the gathered hidden rows; rows whose

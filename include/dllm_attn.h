@@ -274,11 +274,15 @@ int dllm_rope_neox(const dllm_bf16* q_in, int64_t q_in_stride, dllm_bf16* q_out,
  *   x0_p[r] = max_j P_j = bf16(1 / s),  x0[r] = min { j : P_j == x0_p[r] }
  * (torch.max returns the first maximal index).  Rows holding NaN or only
  * -inf give unspecified results (torch's are NaN).  V must be a multiple of
- * 8; logits 16-byte aligned, ld a multiple of 8 and >= V.  One workgroup
- * reduces each row, so dllm_softmax_max_workspace_size returns 0 and
- * workspace may be null (the arguments keep the signature stable).
+ * 8; logits 16-byte aligned, ld a multiple of 8 and >= V.  No workspace is
+ * required (dllm_softmax_max_workspace_size returns 0, null is fine): one
+ * workgroup then reduces each row.  With one of at least
+ * dllm_softmax_max_split_workspace_size(M, V) bytes (device memory, any
+ * contents; 0 where it does not pay) few rows are spread over several
+ * workgroups each.  Calls that may overlap need workspaces of their own.
  */
 size_t dllm_softmax_max_workspace_size(int M, int V);
+size_t dllm_softmax_max_split_workspace_size(int M, int V);
 int dllm_softmax_max(const dllm_bf16* logits, int64_t ld, int M, int V, int64_t* x0, dllm_bf16* x0_p,
                      void* workspace, size_t workspace_bytes, void* stream);
 

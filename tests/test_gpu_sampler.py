@@ -64,6 +64,36 @@ def test_softmax_max_matches_oracle(dev, M, V, sigma, pad):
     _check_k8(bits(full[:, :V]), x0, p)
 
 
+@pytest.mark.parametrize("M,V,sigma,pad,T", [
+    (1, 126464, 2.0, 0, 0.0),        # one row over eight workgroups
+    (20, 16384, 0.3, 0, 0.0),        # ranges merged by the second launch, rescan on every row
+    (3, 8232, 1.0, 8, 0.0),          # 1029 chunks in two ranges, strided
+    (64, 126464, 2.0, 0, 0.0),       # the most rows that are split
+    (5, 33288, 2.0, 8, 1.0),         # noisy: four ranges of 4161 chunks
+    (128, 16392, 2.0, 0, 0.5),       # noisy: the most rows that are split
+])
+def test_softmax_max_split_rows(dev, M, V, sigma, pad, T):
+    """Rows spread over several workgroups (a workspace given) against the
+    oracle, and the same call with a null and a short workspace."""
+    print(f"softmax_max split M={M} V={V} sigma={sigma} pad={pad} T={T}", flush=True)
+    full = (torch.randn(M, V + pad, generator=torch.Generator().manual_seed(V)) * sigma).to(torch.bfloat16)
+    full[:, V:] = 100.0                              # padding columns must be ignored
+    logits = full.to(dev)[:, :V]
+    temps = torch.full((M,), T, dtype=torch.float64, device=dev)
+    need = _capi.softmax_max_split_workspace_size(M, V)
+    assert need > 0
+    for nbytes in (need, need - 1, 0):
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+        x0 = torch.full((M,), -1, dtype=torch.int64, device=dev)
+        p = torch.zeros(M, dtype=torch.bfloat16, device=dev)
+        if T:
+            _capi.softmax_max_sample(logits, temps, 31, 2, x0, p, ws)
+            _check_sample(bits(full[:, :V]), np.full(M, T), 31, 2, x0.cpu().numpy(), bits(p))
+        else:
+            _capi.softmax_max(logits, x0, p, ws)
+            _check_k8(bits(full[:, :V]), x0.cpu().numpy(), bits(p))
+
+
 def test_softmax_max_ties_and_neg_inf(dev):
     print("softmax_max ties / -inf", flush=True)
     V = 126464

@@ -79,6 +79,14 @@ SIGNATURES = {
 _lib = None
 _lock = threading.Lock()
 
+# Host fast paths over the same library (csrc/native.cpp, built beside it).  Each
+# returns None for whatever it does not take; without the module the Python
+# forms serve every call.
+try:
+    from . import _native as native
+except ImportError:
+    native = None
+
 
 def load(path: str | None = None) -> ctypes.CDLL:
     """Load (once) and return the library; raise RuntimeError if it is absent."""

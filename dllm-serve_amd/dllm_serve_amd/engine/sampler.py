@@ -94,12 +94,18 @@ class RemaskSampler:
         drawn from (seed, row index)."""
         M = rows.shape[0]
         dev = rows.device
+        step = M if not self.max_logprobs else self.max_logprobs
+        whole = None
+        if step == M and M and row_temperature is None and _capi.native is not None:
+            whole = self.compute_logits(rows)
+            got = _capi.native.softmax_max(whole)
+            if got is not None and got[0].shape[0] == M:
+                return got
         x0 = torch.empty(M, dtype=torch.int64, device=dev)
         x0_p = torch.empty(M, dtype=torch.bfloat16, device=dev)
-        step = M if not self.max_logprobs else self.max_logprobs
         for a in range(0, M, max(step, 1)):
             b = min(M, a + step)
-            logits = self.compute_logits(rows[a:b])
+            logits = self.compute_logits(rows[a:b]) if whole is None else whole
             if logits.dtype != torch.bfloat16 or logits.dim() != 2 or logits.stride(-1) != 1:
                 raise ValueError("compute_logits must return [rows, vocab] bf16 with a contiguous last dim")
             ws = self._workspace(b - a, logits.shape[1], dev)
@@ -179,10 +185,14 @@ def sample_device_windows(sampler: "RemaskSampler", hidden_states: torch.Tensor,
     """The sampling step with windows built on the device (dllm_step_build's
     smp_rows / smp_params): nothing is computed or copied on the host."""
     n_seq = smp_params.shape[0]
-    n_unmasked = torch.zeros(n_seq, dtype=torch.int32, device=hidden_states.device)
     if smp_rows.numel() == 0:
-        return n_unmasked
+        return torch.zeros(n_seq, dtype=torch.int32, device=hidden_states.device)
     x0, x0_p = sampler.logits_max(hidden_states.index_select(0, smp_rows))
+    if _capi.native is not None:
+        n = _capi.native.unmask(tokens, smp_params, max_win, x0, x0_p, sampler.mask_token_id)
+        if n is not None:
+            return n
+    n_unmasked = torch.zeros(n_seq, dtype=torch.int32, device=hidden_states.device)
     _capi.lowconf_unmask(tokens.view(-1), smp_params, n_seq, max_win, x0, x0_p, sampler.mask_token_id, n_unmasked)
     return n_unmasked
 

@@ -23,6 +23,7 @@ current HIP stream; nothing falls back to the CPU.
 from __future__ import annotations
 
 import os
+import struct
 import weakref
 
 import numpy as np
@@ -244,6 +245,7 @@ class StepPlan:
             setattr(self, k, getattr(lay, k))
         self._ws = {}
         self._args = {}
+        self._packed = {}
         self.last_idx = None
 
     @classmethod
@@ -285,6 +287,13 @@ class StepPlan:
                      ws=None if ws is None else ws.data_ptr(), ws_bytes=0 if ws is None else ws.numel(),
                      ws_tensor=ws)
             self._args[key] = a
+            if not (self.any_skipped or self.n_job) and self.device.type == "cuda":
+                # the step's launches for the native form (csrc/native.cpp, PlanArgs)
+                dev = self.device.index if self.device.index is not None else torch.cuda.current_device()
+                self._packed[key] = struct.pack(
+                    "=17q", dev, self.total_rows, Hq, Hkv, D, self.n_dense, self.max_q_dense, a["cu"],
+                    a["dense_ids"] or 0, self.n_cached, self.max_q_cached, self.max_keys_cached, a["cached_ids"] or 0,
+                    a["slots"], a["slot_off"], a["ws"] or 0, a["ws_bytes"])
         return a
 
 
@@ -314,6 +323,14 @@ class Attention(nn.Module):
         # take that view
         context = get_context()
         if context.is_diffusion:
+            # a step whose plan is built and that only attends: one native call
+            plan = getattr(context, "_dllm_plan", None)
+            if plan is not None and _capi.native is not None:
+                packed = plan._packed.get((self.num_heads, self.num_kv_heads, self.head_dim))
+                if packed is not None:
+                    o = _capi.native.attn(q, k, v, self.k_cache, self.v_cache, packed, float(self.scale))
+                    if o is not None:
+                        return o
             return self._mixed_sparse_dense_attention(q, k, v, context)
         raise NotImplementedError(
             "only the diffusion branch (context.is_diffusion=True) is provided; the autoregressive "

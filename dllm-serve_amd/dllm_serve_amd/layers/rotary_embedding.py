@@ -56,8 +56,12 @@ class RotaryEmbedding(nn.Module):
 
     def forward(self, positions: torch.Tensor, query: torch.Tensor,
                 key: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
-        n = positions.size(0)
         D = self.head_size
+        if _capi.native is not None:
+            out = _capi.native.rope(positions, query, key, self.cos_sin_cache, D, self.inplace)
+            if out is not None:
+                return out
+        n = positions.size(0)
         if self.cos_sin_cache.device != query.device:
             self.cos_sin_cache = self.cos_sin_cache.to(query.device)
         pos = positions if positions.dtype == torch.int64 else positions.to(torch.int64)

@@ -1197,9 +1197,15 @@ extern "C" int dllm_attn_varlen_fwd(const dllm_bf16* q, const dllm_bf16* k, cons
 // against 732 keys: 448 -> 256 workgroups, 28 -> 19.5 us); otherwise 1,
 // which streams the same bytes with twice the workgroups (4 x 32 heads x 2 M
 // tiles against 672 keys: 16.5 us, against 19.3 us paired on 128 CUs).
-// Then the keys are split, only while the splits still fit in one
-// generation (each split adds a partial record and the combine launch), with
-// at least two 128-key tiles per split.
+// Then the keys of more than six 128-key tiles are split, only while the splits
+// still fit in one generation and with at least three tiles each: the partial
+// records and the combine launch cost about 4 us, three tiles of a workgroup's
+// stream.  Measured unsplit / split in us: 384 keys, 1 x 32 rows x 32 heads 9.6
+// / 11.9, 4 x 32 10.6 / 15.1; 672 keys, 2 x 64 14.4 / 15.6; 732 keys, 28 / 4
+// heads, 4 x 32 13.4 / 14.8; 1032 keys, 1 x 32, 28 / 4 16.5 / 13.9 (three
+// tiles a split; two 14.2); 1532 keys, 32 heads 22.5 / 16.1 (two tiles 16.7).
+// Up to 32 workgroups gain from six tiles on: 732 keys, 1 x 32 rows x 32 heads
+// 13.8 / 13.4 (three splits of two tiles).
 static int block_cached_plan(int n_seg, int max_q, int max_keys, int Hq, int Hkv, int& mtiles, int& rb,
                              int& n_split, int& keys_per_split) {
   const int g = Hq / Hkv;
@@ -1209,11 +1215,11 @@ static int block_cached_plan(int n_seg, int max_q, int max_keys, int Hq, int Hkv
   rb = (mtiles >= 2 && (pairs1 + 255) / 256 > (pairs2 + 255) / 256) ? 2 : 1;
   const int64_t pairs = rb == 2 ? pairs2 : pairs1;
   int64_t want = pairs > 0 ? 256 / pairs : 1;
-  const int max_split = max_keys > 0 ? (max_keys + 255) / 256 : 1;
+  const int tiles = (max_keys + CK_TILE - 1) / CK_TILE;
+  const int max_split = pairs <= 32 && tiles >= 6 ? (tiles < 9 ? 3 : tiles / 3) : tiles > 6 ? tiles / 3 : 1;
   if (want > max_split) want = max_split;
   if (want < 1) want = 1;
   n_split = (int)want;
-  const int tiles = (max_keys + CK_TILE - 1) / CK_TILE;
   const int tiles_per_split = (tiles + n_split - 1) / n_split;
   keys_per_split = tiles_per_split * CK_TILE;
   if (keys_per_split <= 0) keys_per_split = CK_TILE;

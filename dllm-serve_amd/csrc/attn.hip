@@ -157,6 +157,25 @@ __device__ __forceinline__ void dense_state_init(DenseState<NQ>& st) {
   }
 }
 
+// Raises the reference maximum of the rows whose tile maximum mx exceeds it by
+// more than kLazy, and rescales their state.
+__device__ __forceinline__ void dense_raise_max(float mx, f32x16_t (&oacc)[4], float& m_run, float& l_run, float& thr,
+                                                float& neg_m) {
+  const bool need = mx > thr;
+  if (__builtin_amdgcn_ballot_w64(need)) {
+    const float m_new = need ? mx : m_run;
+    const float alpha = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
+    l_run *= alpha;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) oacc[db][i] *= alpha;
+    m_run = m_new;
+    thr = m_run + kLazy;
+    neg_m = (m_run == -INFINITY) ? 0.f : -m_run;
+  }
+}
+
 // Online-softmax update of one query block from its two S^T key blocks;
 // returns the packed P^T fragments (B operands of O^T += V^T P^T).
 template <int KB, bool MASK>
@@ -175,19 +194,7 @@ __device__ __forceinline__ void dense_softmax(f32x16_t (&sacc)[KB], f32x16_t (&o
       mx = fmaxf(mx, sacc[b][i]);
     }
   mx = pair_max32(mx) * c;
-  const bool need = mx > thr;
-  if (__builtin_amdgcn_ballot_w64(need)) {
-    const float m_new = need ? mx : m_run;
-    const float alpha = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
-    l_run *= alpha;
-#pragma unroll
-    for (int db = 0; db < 4; ++db)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) oacc[db][i] *= alpha;
-    m_run = m_new;
-    thr = m_run + kLazy;
-    neg_m = (m_run == -INFINITY) ? 0.f : -m_run;
-  }
+  dense_raise_max(mx, oacc, m_run, l_run, thr, neg_m);
   // The row sum adds the bf16-rounded numerators, the same values the O^T
   // product consumes; two partial sums (one starting from l_run) keep the
   // dependent chain short.
@@ -314,6 +321,38 @@ __device__ __forceinline__ void dense_tile(const uint8_t* Ks, const uint8_t* Vs,
 #pragma unroll
       for (int q = 0; q < NQ; ++q)
         st.oacc[q][db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, pf[q][cch], st.oacc[q][db], 0, 0, 0);
+    }
+  }
+}
+
+// One wavefront's 32 finished rows to o through its 8 KiB `ot` of LDS, so that
+// every global store writes whole 256-byte rows: lane (lrow, hl) holds, per d
+// block db and quad rq, d = 32 db + 8 rq + 4 hl + 0..3, i.e. half hl of 16-byte
+// chunk 4 db + rq of its row; chunks XOR-swizzled by row; read back, instruction
+// j carries rows 4j .. 4j+3, one 16-byte chunk per lane.
+__device__ __forceinline__ void store_o_rows(const AttnArgs& a, uint8_t* ot, const f32x16_t (&oacc)[4], float inv,
+                                             int qrow0, int hkv, int m0, int M, int lane) {
+  const int lrow = lane & 31, hl = lane >> 5, g = a.g;
+#pragma unroll
+  for (int db = 0; db < 4; ++db)
+#pragma unroll
+    for (int rq = 0; rq < 4; ++rq) {
+      u32x2_t w;
+      w[0] = cvt_pk_bf16(oacc[db][4 * rq + 0] * inv, oacc[db][4 * rq + 1] * inv);
+      w[1] = cvt_pk_bf16(oacc[db][4 * rq + 2] * inv, oacc[db][4 * rq + 3] * inv);
+      const int chunk = 4 * db + rq;
+      *reinterpret_cast<u32x2_t*>(ot + lrow * 256 + ((chunk ^ (lrow & 15)) * 16) + 8 * hl) = w;
+    }
+  const int rsub = lane >> 4, ch = lane & 15;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int r = 4 * j + rsub;
+    const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ot + r * 256 + ((ch ^ (r & 15)) * 16));
+    const int m = m0 + r;
+    if (m < M) {
+      const int tok = m / g;
+      const int head = hkv * g + (m - tok * g);
+      st128(a.o + (int64_t)(qrow0 + tok) * a.o_stride + head * HD + ch * 8, v);
     }
   }
 }
@@ -479,12 +518,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC, OC
   }
 
   if constexpr (NQ == 1) {
-    // O goes through LDS so that every global store writes whole 256-byte
-    // rows: lane (lrow, hl) holds, per d block db and quad rq, d = 32 db +
-    // 8 rq + 4 hl + 0..3, i.e. half hl of 16-byte chunk 4 db + rq of its row.
-    // The wave's 32 rows x 256 bytes land in its own 8 KiB of the (now free)
-    // K/V stages, chunks XOR-swizzled by row; read back, instruction j
-    // carries rows 4j .. 4j+3, one 16-byte chunk per lane.
     // O staging needs NW * 8 KiB (the Q rows, or the front of LDS); the launch gives at least that
     const float l_tot = pair_sum32(st.l_run[0]);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
@@ -498,28 +531,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC, OC
       __syncthreads();
       ot = lds + wave * 8192;
     }
-#pragma unroll
-    for (int db = 0; db < 4; ++db)
-#pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        u32x2_t w;
-        w[0] = cvt_pk_bf16(st.oacc[0][db][4 * rq + 0] * inv, st.oacc[0][db][4 * rq + 1] * inv);
-        w[1] = cvt_pk_bf16(st.oacc[0][db][4 * rq + 2] * inv, st.oacc[0][db][4 * rq + 3] * inv);
-        const int chunk = 4 * db + rq;
-        *reinterpret_cast<u32x2_t*>(ot + lrow * 256 + ((chunk ^ (lrow & 15)) * 16) + 8 * hl) = w;
-      }
-    const int rsub = lane >> 4, ch = lane & 15;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int r = 4 * j + rsub;
-      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ot + r * 256 + ((ch ^ (r & 15)) * 16));
-      const int m = m_base + wave * 32 + r;
-      if (m < M) {
-        const int tok = m / g;
-        const int head = hkv * g + (m - tok * g);
-        st128(a.o + (int64_t)(qrow0 + tok) * a.o_stride + head * HD + ch * 8, v);
-      }
-    }
+    store_o_rows(a, ot, st.oacc[0], inv, qrow0, hkv, m_base + wave * 32, M, lane);
   } else {
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
@@ -540,6 +552,200 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC, OC
       }
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// K3a for launches of about one workgroup per CU (a few short sequences): at one
+// wavefront per SIMD nothing hides a wavefront's own chain K read -> S^T -> row
+// maximum -> exponentials -> V^T read -> O^T, 0.57 us a tile against 0.27 us for
+// its MFMAs alone.  So the wavefront overlaps its own work: S^T of the next tile
+// is computed beside the softmax of this one, and both tiles' operands are read
+// right after the barrier.  The same products, sums and roundings in the same
+// order as attn_dense_kernel with 32-key tiles (bit-equal outputs, so a row does
+// not depend on the batch it is in).  Two tiles of registers: 229-241 VGPRs.
+// NW = 1, 2 or 4 wavefronts of 32 M rows: fewer rows per workgroup while that
+// spreads the rows over more CUs (see dense_plan).
+// 32 heads, K3a before -> now: 1 x 128 tokens 6.8 -> 6.0 us, 1 x 256 9.1 -> 8.0,
+// 1 x 512 13.7 -> 11.8, 1 x 1024 24.4 -> 22.5; with more workgroups per CU the
+// wavefronts overlap each other and this form is slower (4 x 1280 107 -> 113 us).
+
+// Softmax of one tile (s) with S^T of the next one (sn) in between.
+__device__ __forceinline__ void piped_softmax(f32x16_t& s, f32x16_t& sn, const bf16x8_t (&kf)[8],
+                                              const bf16x8_t (&qf)[8], DenseState<1>& st, bf16x8_t (&pf)[2], float c) {
+  // the branch below ends a scheduling region: three of the eight products go before it
+  constexpr int kBefore = 3;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) sn[i] = 0.f;
+#pragma unroll
+  for (int i = 0; i < kBefore; ++i) sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i], sn, 0, 0, 0);
+  float mx = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
+  mx = pair_max32(mx) * c;
+  dense_raise_max(mx, st.oacc[0], st.m_run[0], st.l_run[0], st.thr[0], st.neg_m[0]);
+  float psum[2] = {st.l_run[0], 0.f};
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    u32x4_t pk;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int at = kBefore + 4 * j + w;
+      if (at < 8) sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[at], qf[at], sn, 0, 0, 0);
+      const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * j + 2 * w], c, st.neg_m[0]));
+      const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * j + 2 * w + 1], c, st.neg_m[0]));
+      pk[w] = cvt_pk_bf16(p0, p1);
+      psum[w & 1] = add_bf16x2(pk[w], psum[w & 1]);
+    }
+    pf[j] = as_bf16x8(pk);
+  }
+  st.l_run[0] = psum[0] + psum[1];
+}
+
+template <int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_dense_piped_kernel(AttnArgs a) {
+  constexpr int TILE = 32 * 256;     // K or V bytes of a tile
+  constexpr int PER_WAVE = 8 / NW;   // DMA instructions of one matrix per wavefront and tile
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  uint8_t* const kst = lds;             // two K tiles
+  uint8_t* const vst = lds + 2 * TILE;  // two V tiles
+  const int L = xcd_remap(blockIdx.x, a.xcd_chunk);
+  if (L >= a.logical_blocks) return;
+  int r = L;
+  const int mt = r % a.mtiles;
+  r /= a.mtiles;
+  const int hkv = r % a.Hkv;
+  const int s = r / a.Hkv;
+  const int sid = a.seg_ids ? a.seg_ids[s] : s;
+  const int qrow0 = a.cu_q[sid];
+  const int Lq = a.cu_q[sid + 1] - qrow0;
+  const int krow0 = a.cu_k[sid];
+  const int Lk = a.cu_k[sid + 1] - krow0;
+  const int g = a.g;
+  const int M = Lq * g;
+  const int m_base = mt * 32 * NW;
+  if (m_base >= M) return;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int hl = lane >> 5;
+  const uint32_t kS = (uint32_t)(a.k_stride * 2), vS = (uint32_t)(a.v_stride * 2);
+  const uint16_t* kseg = a.k + (int64_t)krow0 * a.k_stride + hkv * HD;
+  const uint16_t* vseg = a.v + (int64_t)krow0 * a.v_stride + hkv * HD;
+  DenseAddr ad;
+  dense_addr(ad, lane, kS, vS);
+  // Tile t of a matrix into its stage `par`; only tiles that exist are issued,
+  // rows past the segment read as zero (see attn_dense_kernel).
+  auto issue_k = [&](int t, int par) {
+    const __amdgpu_buffer_rsrc_t rs =
+        make_rsrc(kseg + (int64_t)t * 32 * a.k_stride, (uint32_t)(Lk - 1 - t * 32) * kS + HD * 2);
+#pragma unroll
+    for (int j = 0; j < PER_WAVE; ++j) {
+      const int q = PER_WAVE * wave + j;
+      dma16(rs, kst + par * TILE + q * 1024,
+            (uint32_t)(4 * q) * kS + ad.kdma_row + (ad.kdma_chunk ^ (uint32_t)(64 * (q & 3))));
+    }
+  };
+  auto issue_v = [&](int t, int par) {
+    const __amdgpu_buffer_rsrc_t rs =
+        make_rsrc(vseg + (int64_t)t * 32 * a.v_stride, (uint32_t)(Lk - 1 - t * 32) * vS + HD * 2);
+#pragma unroll
+    for (int j = 0; j < PER_WAVE; ++j) {
+      const int q = PER_WAVE * wave + j;
+      dma16(rs, vst + par * TILE + q * 1024, (uint32_t)(4 * q) * vS + ad.vdma);
+    }
+  };
+  auto read_k = [&](int par, bf16x8_t (&kf)[8]) {
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk)
+      kf[kk] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(kst + par * TILE + (ad.kbase ^ (uint32_t)(32 * kk))));
+  };
+  auto read_v = [&](int par, u32x2_t (&vr)[16]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {  // key chunk i / 4, d block i % 4
+      const uint8_t* vp = vst + par * TILE + (ad.vbase ^ (uint32_t)(64 * (i & 3))) + (i >> 2) * 16 * 256;
+      vr[2 * i] = ds_read_tr16(vp);
+      vr[2 * i + 1] = ds_read_tr16(vp + 8 * 256);
+    }
+  };
+
+  bf16x8_t qf[8];
+  {
+    const uint32_t qS = (uint32_t)(a.q_stride * 2);
+    const uint32_t qbytes = Lq > 0 ? (uint32_t)Lq * qS : 0u;
+    const __amdgpu_buffer_rsrc_t qrs = make_rsrc(a.q + (int64_t)qrow0 * a.q_stride, qbytes);
+    const int m = m_base + wave * 32 + (lane & 31);
+    const int tok = m / g;
+    const uint32_t qoff =
+        m < M ? (uint32_t)tok * qS + (uint32_t)((hkv * g + m - tok * g) * HD + hl * 8) * 2u : qbytes;
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) qf[kk] = as_bf16x8(bload(qrs, qoff + (uint32_t)kk * 32u, 0u));
+  }
+  DenseState<1> st;
+  dense_state_init(st);
+  const float c = a.scale_log2;
+  const int nt = (Lk + 31) / 32;
+  if (nt > 0) {
+    asm volatile("" ::: "memory");  // q first: its wait leaves the tiles in flight
+    issue_k(0, 0);
+    if (nt > 1) issue_k(1, 1);
+    issue_v(0, 0);
+    if (nt > 1) vm_wait<2 * PER_WAVE>(); else vm_wait<PER_WAVE>();  // K(0)
+    lds_barrier();
+    f32x16_t sa, sb;
+    {
+      bf16x8_t kf[8];
+      read_k(0, kf);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sa[i] = 0.f;
+#pragma unroll
+      for (int kk = 0; kk < 8; ++kk) sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kk], qf[kk], sa, 0, 0, 0);
+    }
+    auto add_pv = [&](const u32x2_t (&vr)[16], const bf16x8_t (&pf)[2]) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        st.oacc[0][i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            as_bf16x8(u32x4_t{vr[2 * i][0], vr[2 * i][1], vr[2 * i + 1][0], vr[2 * i + 1][1]}), pf[i >> 2],
+            st.oacc[0][i & 3], 0, 0, 0);
+    };
+    // Tile t (S^T in s0, V in stage par) with S^T of tile t + 1 into s1.  All
+    // reads of a turn come right after its barrier, so the stages read in the
+    // turn before are free: K(t + 2) and V(t + 1) go there.
+    auto turn = [&](f32x16_t& s0, f32x16_t& s1, int t, int par) {
+      vm_wait<0>();  // K(t + 1), V(t)
+      lds_barrier();
+      bf16x8_t kf[8], pf[2];
+      u32x2_t vr[16];
+      read_k(par ^ 1, kf);
+      read_v(par, vr);
+      asm volatile("" ::: "memory");
+      if (t + 2 < nt) issue_k(t + 2, par);
+      issue_v(t + 1, par ^ 1);
+      piped_softmax(s0, s1, kf, qf, st, pf, c);
+      add_pv(vr, pf);
+    };
+    int t = 0;
+    for (; t + 2 < nt; t += 2) {  // two turns: S^T changes registers instead of being copied
+      turn(sa, sb, t, 0);
+      turn(sb, sa, t + 1, 1);
+    }
+    if (t + 1 < nt) {
+      turn(sa, sb, t, 0);
+      sa = sb;
+    }
+    vm_wait<0>();
+    lds_barrier();
+    u32x2_t vr[16];
+    bf16x8_t pf[2];
+    read_v((nt - 1) & 1, vr);
+    f32x16_t last[1] = {sa};
+    dense_softmax<1, true>(last, st.oacc[0], st.m_run[0], st.l_run[0], st.thr[0], st.neg_m[0], pf, c,
+                           Lk - (nt - 1) * 32, 0, hl);
+    add_pv(vr, pf);
+  }
+  const float l_tot = pair_sum32(st.l_run[0]);
+  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  lds_barrier();  // every wavefront is done with the stages
+  store_o_rows(a, lds + wave * 8192, st.oacc[0], inv, qrow0, hkv, m_base + wave * 32, M, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -1095,11 +1301,12 @@ static int set_lds(KernelFn fn, int bytes, const char* name) {
 
 using namespace dllm;
 
-// K3a launch shape: wavefronts per workgroup (4, 12 or 8), keys per tile,
+// K3a launch shape: wavefronts per workgroup (1, 2 or 4 piped, 4, 12 or 8), keys per tile,
 // M tiles per (segment, KV head), XCD chunk and grid.  One function for the
 // launch and for dllm_attn_varlen_launch_shape, so that the two cannot drift.
 struct DensePlan {
   int nw, tk, mtiles, xcd_chunk, grid;
+  bool piped;  // attn_dense_piped_kernel (nw = 1, 2 or 4)
   int64_t logical;
 };
 static DensePlan dense_plan(int n_seg, int max_seqlen_q, int max_seqlen_k, int Hq, int Hkv) {
@@ -1116,6 +1323,20 @@ static DensePlan dense_plan(int n_seg, int max_seqlen_q, int max_seqlen_k, int H
   const bool one_wg = !wide && m_rows > 256 && m_rows <= 384 && (int64_t)n_seg * Hkv >= kOneWgMinPairs;
   p.nw = wide ? 8 : (one_wg ? 12 : 4);
   p.tk = wide ? 64 : 32;
+  // Launches that leave about one wavefront per SIMD: the form that overlaps a
+  // wavefront's own phases, its workgroups as small as one per CU allows.  With
+  // 32 heads, in us, 4 wavefronts plain / piped with 4, 2, 1: 1 x 256 tokens
+  // 9.1 / 9.0, 8.2, 8.0; 1 x 512 13.7 / 13.0, 11.8, 12.7; 1 x 640 16.2 / 15.3,
+  // 19.3, 16.3; 4 x 256 10.5 / 10.2, 12.4, 11.6.  Four wavefronts up to three
+  // workgroups on two CUs: 1 x 1280 (320 workgroups) 40.0 / 38.5, 4 x 384 (384)
+  // 19.1 / 19.0, 8 x 384 as 768 29 / 30 (not taken).
+  if (!wide) {
+    const int64_t pairs = (int64_t)n_seg * Hkv;
+    auto groups = [&](int nw) { return pairs * ((m_rows + 32 * nw - 1) / (32 * nw)); };
+    const int nw = groups(1) <= 256 ? 1 : groups(2) <= 256 ? 2 : groups(4) <= 384 ? 4 : 0;
+    p.piped = nw > 0;
+    if (nw) p.nw = nw;
+  }
   const int bm = 32 * p.nw;
   p.mtiles = (int)((m_rows + bm - 1) / bm);
   p.logical = (int64_t)p.mtiles * Hkv * n_seg;
@@ -1177,7 +1398,9 @@ extern "C" int dllm_attn_varlen_fwd(const dllm_bf16* q, const dllm_bf16* k, cons
   // Measured: the 4-wavefront shape is 5-12 % faster up to 1280 keys
   // (4 x 1280, Dream GQA varlen with up to 1245 keys), the 8-wavefront one
   // 6 % faster at 4096 keys.
-  auto kern = wide ? attn_dense_kernel<8, 1, DENSE_ST, 64, 2>
+  auto kern = plan.piped ? (nw == 1 ? attn_dense_piped_kernel<1>
+                                    : nw == 2 ? attn_dense_piped_kernel<2> : attn_dense_piped_kernel<4>)
+              : wide ? attn_dense_kernel<8, 1, DENSE_ST, 64, 2>
                    : (one_wg ? attn_dense_kernel<12, 1, DENSE_ST, 32, 3> : attn_dense_kernel<4, 1, DENSE_ST, 32, 3>);
   int lds_bytes = DENSE_ST * 2 * (wide ? 64 : 32) * 256;
   if (wide || one_wg)

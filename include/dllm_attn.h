@@ -98,7 +98,7 @@ int dllm_attn_varlen_fwd(const dllm_bf16* q, const dllm_bf16* k, const dllm_bf16
 
 /*
  * Launch shape dllm_attn_varlen_fwd picks for these sizes, without launching:
- * wavefronts per workgroup (4, 12 or 8), keys per LDS tile and the grid (0
+ * wavefronts per workgroup (1, 2, 4, 8 or 12), keys per LDS tile and the grid (0
  * when there is nothing to do).  No counterpart in the reference (flash-attn
  * chooses its tiling internally); it lets tests and profiles name the kernel
  * a given call runs.  Any output pointer may be null.

@@ -375,3 +375,46 @@ def test_block_cached_invalid_slots_are_excluded(dev, Hq, Hkv):
         ref = oatt.block_cached(to_np(q)[r0:r1], to_np(k)[r0:r1], to_np(v)[r0:r1], to_np(kc), to_np(vc), slots[i],
                                 D ** -0.5, dtype=np.float32)
         assert_attn_close(o[r0:r1], ref, f"seq {i}")
+
+
+@pytest.mark.parametrize("Hq,Hkv,lq,lk,wavefronts", [
+    (4, 4, 33, 1, 1),        # one key: no turn of the tile loop
+    (4, 4, 31, 33, 1),       # two tiles, the last of one key
+    (4, 4, 64, 64, 1),
+    (28, 4, 9, 97, 1),       # grouped heads, rows past the segment in the row block
+    (32, 32, 257, 95, 2),    # 9 row blocks of 32 per head: 288 workgroups of one
+    (32, 32, 512, 512, 2),
+    (32, 32, 513, 160, 4),
+    (28, 4, 800, 129, 4),
+    (4, 4, 40, 0, 1),        # no keys: zero rows
+])
+def test_piped_launch_rows_equal_a_batch(dev, Hq, Hkv, lq, lk, wavefronts):
+    """Launches of about one workgroup per CU overlap a wavefront's own phases;
+    their rows are bit-equal to the same segment inside a batch that runs the
+    plain form, and match the oracle; strided rows."""
+    print(f"piped dense Hq={Hq} Hkv={Hkv} lq={lq} lk={lk}", flush=True)
+    D = 128
+    assert _capi.varlen_launch_shape(1, lq, max(lk, 1), Hq, Hkv, D)["wavefronts"] == wavefronts
+    copies = 130 if lq <= 128 else 14
+    g = torch.Generator(device=dev).manual_seed(lq * 7 + lk)
+    q = torch.randn(lq, (Hq + 1) * D + 8, generator=g, device=dev).bfloat16()[:, :Hq * D].unflatten(1, (Hq, D))
+    k = torch.randn(max(lk, 1), Hkv * D + 24, generator=g, device=dev).bfloat16()[:, :Hkv * D].unflatten(1, (Hkv, D))
+    v = torch.randn(max(lk, 1), Hkv, D, generator=g, device=dev).bfloat16()
+    cu_q = torch.tensor([0, lq], dtype=torch.int32, device=dev)
+    cu_k = torch.tensor([0, lk], dtype=torch.int32, device=dev)
+    o = torch.full((lq, Hq, D), float("nan"), dtype=torch.bfloat16, device=dev)
+    _capi.attn_varlen_fwd(q, k, v, o, cu_q, cu_k, None, 1, lq, D ** -0.5, max_seqlen_k=lk)
+    if lk == 0:
+        assert torch.all(o == 0)
+        return
+    rep = [x.repeat(copies, 1, 1).contiguous() for x in (q, k, v)]
+    assert _capi.varlen_launch_shape(copies, lq, lk, Hq, Hkv, D)["wavefronts"] in (4, 12)
+    ob = torch.empty(copies * lq, Hq, D, dtype=torch.bfloat16, device=dev)
+    _capi.attn_varlen_fwd(*rep, ob, (torch.arange(copies + 1, device=dev) * lq).int(),
+                          (torch.arange(copies + 1, device=dev) * lk).int(), None, copies, lq, D ** -0.5,
+                          max_seqlen_k=lk)
+    torch.cuda.synchronize()
+    for i in (0, copies - 1):
+        assert torch.equal(ob[i * lq:(i + 1) * lq].view(torch.int16), o.view(torch.int16)), i
+    ref = oatt.varlen(to_np(q), to_np(k), to_np(v), [0, lq], [0, lk], D ** -0.5, dtype=np.float32)
+    assert_attn_close(o, ref, "piped")

@@ -255,6 +255,40 @@ __device__ __forceinline__ void v_operands_untracked(const uint8_t* Vs, const De
       : "memory");
 }
 
+// The same for NDB d blocks from vb (vbase with the first block's 64 d XORed in);
+// output index (NDB c + d) * 2 + h.
+template <int NDB>
+__device__ __forceinline__ void v_operands_blocks(const uint8_t* Vs, uint32_t vb, u32x2_t (&r)[4 * NDB]) {
+  static_assert(NDB == 1 || NDB == 2, "d blocks");
+  const uint32_t b0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)(Vs + vb);
+  if constexpr (NDB == 1) {
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %4\n"
+        "ds_read_b64_tr_b16 %1, %4 offset:2048\n"
+        "ds_read_b64_tr_b16 %2, %4 offset:4096\n"
+        "ds_read_b64_tr_b16 %3, %4 offset:6144\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])
+        : "v"(b0)
+        : "memory");
+  } else {
+    const uint32_t b1 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)(Vs + (vb ^ 64u));
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %8\n"
+        "ds_read_b64_tr_b16 %1, %8 offset:2048\n"
+        "ds_read_b64_tr_b16 %2, %9\n"
+        "ds_read_b64_tr_b16 %3, %9 offset:2048\n"
+        "ds_read_b64_tr_b16 %4, %8 offset:4096\n"
+        "ds_read_b64_tr_b16 %5, %8 offset:6144\n"
+        "ds_read_b64_tr_b16 %6, %9 offset:4096\n"
+        "ds_read_b64_tr_b16 %7, %9 offset:6144\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7])
+        : "v"(b0), "v"(b1)
+        : "memory");
+  }
+}
+
 template <int NQ, int TK, bool MASK, bool UNTRACKED_V = false>
 __device__ __forceinline__ void dense_tile(const uint8_t* Ks, const uint8_t* Vs, const DenseAddr& ad,
                                            const bf16x8_t (&qf)[NQ][8], DenseState<NQ>& st, float c, int k_valid,
@@ -786,10 +820,14 @@ __device__ __forceinline__ void gdma16(const void* g, uint8_t* lds_dst) {
 // (row q, d0 .. d0 + 15) of each row block merges its four partials,
 // wavefronts in order, each scaled term (and each term of the row sum)
 // rounded before it is added.
-template <int RB>
+template <int RB, int DS>
 __device__ __forceinline__ void cached_merge_store(const AttnArgs& a, uint8_t* lds, int last_stage, float* ring,
                                                         const DenseState<1>& st, int s, int hkv, int mt, int split,
-                                                        int qrow0, int M, int m_base, int g, int tid, int rblk) {
+                                                        int qrow0, int M, int m_base, int g, int tid, int rblk,
+                                                        int dpart) {
+  constexpr int NDB = 4 / DS;     // d blocks of 32 this workgroup owns
+  constexpr int DPT = 16 / DS;    // d positions a thread merges
+  const int dbase = dpart * 32 * NDB;
   const int wave = (tid >> 6) & 3;
   const int lane = tid & 63;
   const int lrow = lane & 31;
@@ -804,7 +842,7 @@ __device__ __forceinline__ void cached_merge_store(const AttnArgs& a, uint8_t* l
   }
   auto park = [&]() {
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+    for (int db = 0; db < NDB; ++db)
 #pragma unroll
       for (int rq = 0; rq < 4; ++rq) {
         const int d = db * 32 + 8 * rq + 4 * hl;
@@ -822,7 +860,7 @@ __device__ __forceinline__ void cached_merge_store(const AttnArgs& a, uint8_t* l
   lds_barrier();
   tid &= 255;
   const int q = tid & 31;
-  const int d0 = (tid >> 5) * 16;
+  const int d0 = (tid >> 5) * DPT;  // inside the workgroup's d range
   float mw[4], mq = -INFINITY;
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
@@ -831,16 +869,16 @@ __device__ __forceinline__ void cached_merge_store(const AttnArgs& a, uint8_t* l
   }
   const float mq_use = (mq == -INFINITY) ? 0.f : mq;
   float lq = 0.f;
-  float acc[16];
+  float acc[DPT];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  for (int i = 0; i < DPT; ++i) acc[i] = 0.f;
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
     const float f = (mw[w] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw[w] - mq_use);
     lq = __fadd_rn(lq, __fmul_rn(ml[(w * 2 + 1) * 32 + q], f));  // f = 0 for a wavefront without keys
     const uint8_t* row = part + (d0 >> 6) * CK_TILE * 256 + (w * 32 + q) * 256;
 #pragma unroll
-    for (int c4 = 0; c4 < 4; ++c4) {
+    for (int c4 = 0; c4 < DPT / 4; ++c4) {
       const f32x4_t v = *reinterpret_cast<const f32x4_t*>(row + (((((d0 & 63) >> 2) + c4) ^ (q & 15)) << 4));
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[4 * c4 + e] = __fadd_rn(acc[4 * c4 + e], __fmul_rn(v[e], f));
@@ -852,24 +890,26 @@ __device__ __forceinline__ void cached_merge_store(const AttnArgs& a, uint8_t* l
     const int hq = hkv * g + (mrow - tq * g);
     if (a.n_split == 1) {
       const float inv = lq > 0.f ? 1.f / lq : 0.f;
-      uint16_t* op = a.o + (int64_t)(qrow0 + tq) * a.o_stride + hq * HD + d0;
-      u32x4_t w0, w1;
+      uint16_t* op = a.o + (int64_t)(qrow0 + tq) * a.o_stride + hq * HD + dbase + d0;
+      uint32_t w[DPT / 2];
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        w0[w] = cvt_pk_bf16(acc[2 * w] * inv, acc[2 * w + 1] * inv);
-        w1[w] = cvt_pk_bf16(acc[8 + 2 * w] * inv, acc[8 + 2 * w + 1] * inv);
+      for (int i = 0; i < DPT / 2; ++i) w[i] = cvt_pk_bf16(acc[2 * i] * inv, acc[2 * i + 1] * inv);
+      if constexpr (DPT == 4) {
+        *reinterpret_cast<u32x2_t*>(op) = u32x2_t{w[0], w[1]};
+      } else {
+#pragma unroll
+        for (int i = 0; i < DPT / 8; ++i)
+          st128(op + 8 * i, u32x4_t{w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]});
       }
-      st128(op, w0);
-      st128(op + 8, w1);
     } else {
       const int64_t Prec = (((int64_t)s * a.Hkv + hkv) * a.mtiles + mt) * a.n_split + split;
-      float* po = a.ws + (Prec * 32 + q) * HD + d0;
+      float* po = a.ws + (Prec * 32 + q) * HD + dbase + d0;
 #pragma unroll
-      for (int i = 0; i < 16; i += 4) {
+      for (int i = 0; i < DPT; i += 4) {
         f32x4_t v4 = {acc[i], acc[i + 1], acc[i + 2], acc[i + 3]};
         *reinterpret_cast<f32x4_t*>(po + i) = v4;
       }
-      if (d0 == 0) {  // one writer per row
+      if (d0 == 0 && dpart == 0) {  // one writer per row
         const int64_t nrec = (int64_t)a.n_seg * a.Hkv * a.mtiles * a.n_split;
         float* pml = a.ws + nrec * 32 * HD + (Prec * 32 + q) * 2;
         pml[0] = mq;
@@ -882,6 +922,7 @@ __device__ __forceinline__ void cached_merge_store(const AttnArgs& a, uint8_t* l
 // One 32-key block of the four-wavefront K3b: K operands from LDS, keys set in
 // `bad` left out of the softmax by a small conditional block (a single
 // softmax code path keeps the accumulators in place).
+template <int DS>
 __device__ __forceinline__ void cached_tile(const uint8_t* Ks, const uint8_t* Vs, const DenseAddr& ad,
                                             const bf16x8_t (&qf)[1][8], DenseState<1>& st, float c, uint64_t bad) {
   const int hl = (threadIdx.x & 63) >> 5;
@@ -904,13 +945,17 @@ __device__ __forceinline__ void cached_tile(const uint8_t* Ks, const uint8_t* Vs
   // all 16 V^T operands are read (one asm block) before the first product:
   // the MFMAs read their source registers after issue, so no register they
   // use may be rewritten by a later LDS read while they run
-  u32x2_t vr[16];
-  v_operands_untracked(Vs, ad, vr);
+  constexpr int NDB = 4 / DS;
+  u32x2_t vr[4 * NDB];
+  if constexpr (DS == 1)
+    v_operands_untracked(Vs, ad, vr);
+  else
+    v_operands_blocks<NDB>(Vs, ad.vbase, vr);  // vbase already holds the first block
 #pragma unroll
   for (int cch = 0; cch < 2; ++cch)
 #pragma unroll
-    for (int db = 0; db < 4; ++db) {
-      const u32x2_t lo = vr[(4 * cch + db) * 2], hi = vr[(4 * cch + db) * 2 + 1];
+    for (int db = 0; db < NDB; ++db) {
+      const u32x2_t lo = vr[(NDB * cch + db) * 2], hi = vr[(NDB * cch + db) * 2 + 1];
       st.oacc[0][db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(u32x4_t{lo[0], lo[1], hi[0], hi[1]}), pf[cch],
                                                                st.oacc[0][db], 0, 0, 0);
     }
@@ -936,7 +981,13 @@ __device__ __forceinline__ void cached_tile(const uint8_t* Ks, const uint8_t* Vs
 // its first memory operation -- no wavefront waits for another -- so its first
 // K/V tiles wait on one round of loads (page ids, offsets and Q together)
 // instead of two (slot offsets, then the slot list).
-template <int RB, bool PAGED>
+// DS > 1: the output's d positions are dealt to DS workgroups, each computing
+// the whole S^T and softmax but reading V, and writing O, of 128 / DS positions
+// only (the same values: a d position's sum does not depend on the others).  A
+// CU takes in 26-50 KB a microsecond however idle the chip is, so a launch of
+// few workgroups is bound by each one's bytes: 1 - (1 - 1 / DS) / 2 of them are
+// left (K again from the L2 they share), without partials to merge.
+template <int RB, bool PAGED, int DS>
 // The launch geometry and the tables the first, dependent loads read come as
 // leading scalar arguments (14 dwords): the library is built with kernel
 // argument preloading, so they are in SGPRs when a wave starts instead of one
@@ -956,6 +1007,8 @@ __global__ __launch_bounds__(256 * RB) __attribute__((amdgpu_waves_per_eu(2, 2))
   if (L >= logical_blocks) return;
   const int mblocks = (mtiles + RB - 1) / RB;
   int r = L;
+  const int dpart = DS > 1 ? r % DS : 0;
+  if (DS > 1) r /= DS;
   const int split = r % n_split;
   r /= n_split;
   const int mb = r % mblocks;
@@ -1009,6 +1062,7 @@ __global__ __launch_bounds__(256 * RB) __attribute__((amdgpu_waves_per_eu(2, 2))
   // 32 w + 4j + rl; K chunk (P ^ rl) ^ 4(j & 3), V chunk P ^ 4 rl.
   const uint32_t kchunk = (uint32_t)((P ^ rl) * 16);
   const uint32_t vchunk = (uint32_t)((P ^ (4 * rl)) * 16);
+  const bool v_lane = (P ^ (4 * rl)) / (16 / DS) == dpart;  // this lane's V piece is of the workgroup's d range
   const int64_t row_elems = (int64_t)Hkv * HD;
   // without a cache (cache_slots = 0, slots may be null) every cached row is
   // outside it: the fetches then read slot_off[0], a valid dummy
@@ -1107,7 +1161,8 @@ __global__ __launch_bounds__(256 * RB) __attribute__((amdgpu_waves_per_eu(2, 2))
       const uint64_t vaddr = (use_cache ? vc0 : vb0) + (uint64_t)idx * (use_cache ? cache_row_b : vS_b);
       const int q = 8 * wave + j;
       gdma16(reinterpret_cast<const uint8_t*>(kaddr) + (kchunk ^ (uint32_t)(64 * (jj & 3))), stage + q * 1024);
-      gdma16(reinterpret_cast<const uint8_t*>(vaddr) + vchunk, stage + CK_TILE * 256 + q * 1024);
+      // (the other lanes' pieces belong to another workgroup's d positions)
+      if (DS == 1 || v_lane) gdma16(reinterpret_cast<const uint8_t*>(vaddr) + vchunk, stage + CK_TILE * 256 + q * 1024);
     }
   };
   // keys of this wave's block of tile t whose slot is invalid, as a 32-bit
@@ -1162,6 +1217,7 @@ __global__ __launch_bounds__(256 * RB) __attribute__((amdgpu_waves_per_eu(2, 2))
 
   DenseAddr ad;
   dense_addr(ad, lane, 0u, 0u);
+  ad.vbase ^= (uint32_t)(64 * (4 / DS) * dpart);
   DenseState<1> st;
   dense_state_init(st);
   const float c = a.scale_log2;
@@ -1182,7 +1238,7 @@ __global__ __launch_bounds__(256 * RB) __attribute__((amdgpu_waves_per_eu(2, 2))
     const int k_valid = kend - (k0 + 32 * wave);
     uint64_t badk = bad_t0;
     if (k_valid < 32) badk |= k_valid <= 0 ? 0xffffffffull : (0xffffffffull << k_valid) & 0xffffffffull;
-    cached_tile(cur, cur + CK_TILE * 256, ad, qf, st, c, badk);
+    cached_tile<DS>(cur, cur + CK_TILE * 256, ad, qf, st, c, badk);
     uint32_t bad_t2 = 0;
     if (t + 2 < ntiles) {
       // stage t&1 is free again (with RB > 1 once both row blocks are done
@@ -1198,8 +1254,8 @@ __global__ __launch_bounds__(256 * RB) __attribute__((amdgpu_waves_per_eu(2, 2))
     bad_t0 = bad_t1;
     bad_t1 = bad_t2;
   }
-  cached_merge_store<RB>(a, lds, (ntiles - 1) & 1, reinterpret_cast<float*>(slot_ring), st, s, hkv, mt, split,
-                              qrow0, M, m_base, g, tid, rblk);
+  cached_merge_store<RB, DS>(a, lds, (ntiles - 1) & 1, reinterpret_cast<float*>(slot_ring), st, s, hkv, mt, split,
+                             qrow0, M, m_base, g, tid, rblk, dpart);
 }
 
 // Merge the n_split partial records of every (segment, head, M row).
@@ -1429,8 +1485,14 @@ extern "C" int dllm_attn_varlen_fwd(const dllm_bf16* q, const dllm_bf16* k, cons
 // tiles a split; two 14.2); 1532 keys, 32 heads 22.5 / 16.1 (two tiles 16.7).
 // Up to 32 workgroups gain from six tiles on: 732 keys, 1 x 32 rows x 32 heads
 // 13.8 / 13.4 (three splits of two tiles).
+// Launches that still leave CUs idle deal the output's d positions to 2 or 4
+// workgroups, as many as one generation holds.  Measured with 1 / 2 / 4 in us,
+// caches from HBM: 1 x 32 rows x 32 heads against 352 cached rows 10.1 / 8.9 /
+// 8.4, 2 x 32 10.5 / 9.4 / 8.9, 4 x 32 (128 workgroups) 11.1 / 10.2 / 16.5; 1 x
+// 64 against 608 14.2 / 13.0 / 12.5; 28 / 4 heads, 4 x 32 against 700 13.8 / 12.8
+// / 23.2; 1 x 32 against 1500 (four key splits) 15.9 / 14.6 / 20.8.
 static int block_cached_plan(int n_seg, int max_q, int max_keys, int Hq, int Hkv, int& mtiles, int& rb,
-                             int& n_split, int& keys_per_split) {
+                             int& n_split, int& keys_per_split, int& d_split) {
   const int g = Hq / Hkv;
   mtiles = (max_q * g + 31) / 32;
   const int64_t pairs1 = (int64_t)n_seg * Hkv * mtiles;
@@ -1451,14 +1513,16 @@ static int block_cached_plan(int n_seg, int max_q, int max_keys, int Hq, int Hkv
   // one workspace size serves both)
   if (keys_per_split > 64 * 256 - 256) keys_per_split = 64 * 256 - 256;
   n_split = max_keys > 0 ? (max_keys + keys_per_split - 1) / keys_per_split : 1;
+  const int64_t groups = pairs * n_split;
+  d_split = rb > 1 ? 1 : groups * 4 <= 256 ? 4 : groups * 2 <= 256 ? 2 : 1;
   return 0;
 }
 
 extern "C" size_t dllm_attn_block_cached_workspace_size(int n_seg, int max_q, int max_keys, int Hq, int Hkv, int D) {
   (void)D;
   if (n_seg <= 0 || max_q <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv) return 0;
-  int mtiles, rb, n_split, kps;
-  block_cached_plan(n_seg, max_q, max_keys, Hq, Hkv, mtiles, rb, n_split, kps);
+  int mtiles, rb, n_split, kps, ds;
+  block_cached_plan(n_seg, max_q, max_keys, Hq, Hkv, mtiles, rb, n_split, kps, ds);
   if (n_split <= 1) return 0;
   const size_t nrec = (size_t)n_seg * Hkv * mtiles * n_split;
   return nrec * 32 * (HD + 2) * sizeof(float);
@@ -1468,11 +1532,11 @@ extern "C" int dllm_attn_block_cached_launch_shape(int n_seg, int max_q, int max
                                                    int* row_blocks, int* n_split, int* grid) {
   if (D != HD || Hq <= 0 || Hkv <= 0 || Hq % Hkv || n_seg < 0 || max_q < 0 || max_keys < 0)
     return fail(DLLM_ERR_INVALID_ARG, "dllm_attn_block_cached_launch_shape: unsupported sizes");
-  int mtiles = 0, rb = 1, ns = 1, kps = 0;
-  block_cached_plan(n_seg, max_q, max_keys, Hq, Hkv, mtiles, rb, ns, kps);
+  int mtiles = 0, rb = 1, ns = 1, kps = 0, ds = 1;
+  block_cached_plan(n_seg, max_q, max_keys, Hq, Hkv, mtiles, rb, ns, kps, ds);
   const int mblocks = (mtiles + rb - 1) / rb;
-  const int64_t logical = (int64_t)ns * mblocks * Hkv * n_seg;
-  const int64_t per_pair = (int64_t)ns * mblocks;
+  const int64_t logical = (int64_t)ds * ns * mblocks * Hkv * n_seg;
+  const int64_t per_pair = (int64_t)ds * ns * mblocks;
   const int64_t grain = 8 * (per_pair < 16 ? per_pair : 16);
   if (row_blocks) *row_blocks = rb;
   if (n_split) *n_split = ns;
@@ -1517,8 +1581,8 @@ static int block_cached_impl(const char* name, const dllm_bf16* q, const dllm_bf
   a.cu_q = cu; a.cu_k = cu; a.seg_ids = seg_ids; a.slots = slots; a.slot_off = slot_off;
   a.q_stride = q_stride_tok; a.k_stride = k_stride_tok; a.v_stride = v_stride_tok; a.o_stride = o_stride_tok;
   a.n_seg = n_seg; a.Hkv = Hkv; a.g = Hq / Hkv;
-  int mtiles, rb, n_split, kps;
-  block_cached_plan(n_seg, max_q, max_keys, Hq, Hkv, mtiles, rb, n_split, kps);
+  int mtiles, rb, n_split, kps, ds;
+  block_cached_plan(n_seg, max_q, max_keys, Hq, Hkv, mtiles, rb, n_split, kps, ds);
   a.mtiles = mtiles; a.n_split = n_split; a.keys_per_split = kps;
   if (n_split > 1) {
     const size_t need = dllm_attn_block_cached_workspace_size(n_seg, max_q, max_keys, Hq, Hkv, D);
@@ -1529,14 +1593,14 @@ static int block_cached_impl(const char* name, const dllm_bf16* q, const dllm_bf
     a.ws = reinterpret_cast<float*>(workspace);
   }
   const int mblocks = (mtiles + rb - 1) / rb;
-  const int64_t logical = (int64_t)n_split * mblocks * Hkv * n_seg;
+  const int64_t logical = (int64_t)ds * n_split * mblocks * Hkv * n_seg;
   if (logical > (int64_t)1 << 30) return fail(DLLM_ERR_INVALID_ARG, "%s: problem too large", name);
   a.logical_blocks = (int)logical;
   a.scale_log2 = softmax_scale * kLog2e;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   // one chunk per (segment, KV head): its row blocks and splits read the same
   // cached rows; the pairs of one segment go to all eight XCDs
-  const int64_t per_pair = (int64_t)n_split * mblocks;
+  const int64_t per_pair = (int64_t)ds * n_split * mblocks;
   a.xcd_chunk = (int)(per_pair < 16 ? per_pair : 16);
   const int64_t grain = 8 * (int64_t)a.xcd_chunk;
   const int nb = (int)((logical + grain - 1) / grain * grain);
@@ -1551,12 +1615,17 @@ static int block_cached_impl(const char* name, const dllm_bf16* q, const dllm_bf
                                                       a);
     return DLLM_OK;
   };
+  auto pick = [&](auto slot_form, auto page_form, int threads, int lds_bytes) {
+    return paged ? launch(page_form, threads, lds_bytes) : launch(slot_form, threads, lds_bytes);
+  };
   if (rb == 2)
-    rc = paged ? launch(attn_cached_kernel<2, true>, 512, ck_lds_bytes(2))
-               : launch(attn_cached_kernel<2, false>, 512, ck_lds_bytes(2));
+    rc = pick(attn_cached_kernel<2, false, 1>, attn_cached_kernel<2, true, 1>, 512, ck_lds_bytes(2));
+  else if (ds == 4)
+    rc = pick(attn_cached_kernel<1, false, 4>, attn_cached_kernel<1, true, 4>, 256, ck_lds_bytes(1));
+  else if (ds == 2)
+    rc = pick(attn_cached_kernel<1, false, 2>, attn_cached_kernel<1, true, 2>, 256, ck_lds_bytes(1));
   else
-    rc = paged ? launch(attn_cached_kernel<1, true>, 256, ck_lds_bytes(1))
-               : launch(attn_cached_kernel<1, false>, 256, ck_lds_bytes(1));
+    rc = pick(attn_cached_kernel<1, false, 1>, attn_cached_kernel<1, true, 1>, 256, ck_lds_bytes(1));
   if (rc) return rc;
   if ((rc = check_launch(name))) return rc;
   if (n_split > 1) {

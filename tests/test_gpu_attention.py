@@ -418,3 +418,63 @@ def test_piped_launch_rows_equal_a_batch(dev, Hq, Hkv, lq, lk, wavefronts):
         assert torch.equal(ob[i * lq:(i + 1) * lq].view(torch.int16), o.view(torch.int16)), i
     ref = oatt.varlen(to_np(q), to_np(k), to_np(v), [0, lq], [0, lk], D ** -0.5, dtype=np.float32)
     assert_attn_close(o, ref, "piped")
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("n_seg,Hq,Hkv,lq,nc,parts", [
+    (1, 32, 32, 32, 352, 4),     # 32 workgroups: four per (segment, KV head), 32 d positions each
+    (1, 4, 4, 1, 0, 4),          # one block row, nothing cached
+    (2, 28, 4, 9, 129, 4),       # 63 M rows: a row block with one idle row
+    (3, 32, 32, 20, 257, 2),     # 96 workgroups: two
+    (1, 32, 32, 97, 31, 2),      # four row blocks
+    (4, 32, 32, 32, 608, 2),     # 128 workgroups
+])
+def test_block_cached_d_parts_equal_a_batch(dev, paged, n_seg, Hq, Hkv, lq, nc, parts):
+    """Launches of few workgroups deal the head dim to several of them: the
+    grid says so, and the rows are bit-equal to the same segments inside a
+    batch that fills the chip, and match the oracle."""
+    print(f"block_cached d parts n_seg={n_seg} {Hq}/{Hkv} lq={lq} nc={nc} paged={paged}", flush=True)
+    D = 128
+    pages = -(-nc // 256) + 1
+    copies = max(2, -(-160 // (n_seg * Hkv)))
+    g = torch.Generator(device=dev).manual_seed(nc + lq)
+    q = torch.randn(n_seg * lq, Hq, D, generator=g, device=dev).bfloat16()
+    k, v = (torch.randn(n_seg * lq, Hkv, D, generator=g, device=dev).bfloat16() for _ in range(2))
+    kc, vc = (torch.randn(n_seg * pages * 256, Hkv, D, generator=g, device=dev).bfloat16() for _ in range(2))
+    table = torch.randperm(n_seg * pages, generator=torch.Generator().manual_seed(3)).view(n_seg, pages)
+    rows = torch.arange(nc)
+    slots = table[:, rows // 256] * 256 + rows % 256
+
+    def run(rep):
+        n = n_seg * rep
+        x = [t.repeat(rep, 1, 1).contiguous() for t in (q, k, v)]
+        cu = (torch.arange(n + 1, device=dev) * lq).int()
+        o = torch.full_like(x[0], float("nan"))
+        ws_b = _capi.block_cached_workspace_size(n, lq, nc + lq, Hq, Hkv, D)
+        ws = torch.empty(max(ws_b, 16), dtype=torch.uint8, device=dev)
+        if paged:
+            _capi.attn_block_cached_paged_fwd(*x, o, cu, None, n, lq, nc + lq, kc, vc,
+                                              table.repeat(rep, 1).int().contiguous().to(dev),
+                                              torch.full((n,), nc, dtype=torch.int32, device=dev), D ** -0.5, ws)
+        else:
+            _capi.attn_block_cached_fwd(*x, o, cu, None, n, lq, nc + lq, kc, vc,
+                                        torch.cat([slots.repeat(rep, 1).flatten(), torch.zeros(1)]).int().to(dev),
+                                        (torch.arange(n + 1, device=dev) * nc).int(), D ** -0.5, ws)
+        torch.cuda.synchronize()
+        return o
+
+    shape = _capi.block_cached_launch_shape(n_seg, lq, nc + lq, Hq, Hkv, D)
+    blocks = n_seg * Hkv * -(-(lq * Hq // Hkv) // 32)
+    assert shape["n_split"] == 1 and shape["row_blocks"] == 1 and shape["grid"] >= parts * blocks
+    full = _capi.block_cached_launch_shape(n_seg * copies, lq, nc + lq, Hq, Hkv, D)
+    assert full["n_split"] == 1 and full["grid"] < 2 * copies * blocks + 128
+    alone, batch = run(1), run(copies)
+    for i in (0, copies - 1):
+        part = batch[i * n_seg * lq:(i + 1) * n_seg * lq]
+        assert torch.equal(part.view(torch.int16), alone.view(torch.int16)), i
+    kcn, vcn = to_np(kc), to_np(vc)
+    for s in range(n_seg):
+        sl = slice(s * lq, (s + 1) * lq)
+        ref = oatt.block_cached(to_np(q[sl]), to_np(k[sl]), to_np(v[sl]), kcn, vcn, slots[s].tolist(), D ** -0.5,
+                                dtype=np.float32)
+        assert_attn_close(alone[sl], ref, f"segment {s}")

@@ -325,16 +325,21 @@ class Attention(nn.Module):
         if context.is_diffusion:
             # a step whose plan is built and that only attends: one native call
             plan = getattr(context, "_dllm_plan", None)
-            if plan is not None and _capi.native is not None:
-                packed = plan._packed.get((self.num_heads, self.num_kv_heads, self.head_dim))
-                if packed is not None:
-                    o = _capi.native.attn(q, k, v, self.k_cache, self.v_cache, packed, float(self.scale))
-                    if o is not None:
-                        return o
+            if plan is not None:
+                o = self._native_attention(plan, q, k, v)
+                if o is not None:
+                    return o
             return self._mixed_sparse_dense_attention(q, k, v, context)
         raise NotImplementedError(
             "only the diffusion branch (context.is_diffusion=True) is provided; the autoregressive "
             "prefill/decode branch of the reference is unused by diffusion models")
+
+    def _native_attention(self, plan, q, k, v):
+        """The step's attention through the native form, or None (see csrc/native.cpp)."""
+        packed = plan._packed.get((self.num_heads, self.num_kv_heads, self.head_dim))
+        if packed is None or _capi.native is None:
+            return None
+        return _capi.native.attn(q, k, v, self.k_cache, self.v_cache, packed, float(self.scale))
 
     def _plan(self, context, device) -> StepPlan:
         plan = getattr(context, "_dllm_plan", None)
@@ -378,9 +383,14 @@ class Attention(nn.Module):
         plan = self._plan(context, dev)
         if nq != plan.total_rows or nk != plan.total_rows or nv != plan.total_rows:
             raise ValueError(f"q/k/v have {nq}/{nk}/{nv} rows, the step's sequences feed {plan.total_rows}")
+        first = (Hq, Hkv, D) not in plan._args
+        args = plan.launch_args(Hq, Hkv, D)
+        if first:  # the step's first layer of this shape: its launch arguments exist only now
+            o = self._native_attention(plan, q, k, v)
+            if o is not None:
+                return o
         o = torch.zeros_like(q) if plan.any_skipped else torch.empty_like(q)
         o_st = o.stride(0)
-        args = plan.launch_args(Hq, Hkv, D)
         stream = _capi._stream(dev)
         qp, kp, vp, op = q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr()
 

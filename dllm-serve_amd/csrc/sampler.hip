@@ -138,26 +138,40 @@ __device__ __forceinline__ void smx_batch(const u32x4_t (&v)[U], int c, int step
 // is not the maximum.  A cheap bound tells most of them: with h = the high 32
 // bits of the draw, E >= 1 - u > (2^32 - 1 - h) 2^-32, hence
 //   log2 v < l log2(e) - T (log2(2^32 - 1 - h) - 32).
-// The wavefront keeps a threshold from the largest value any of its lanes has
-// computed; a logit whose bound is below it is left out, all others (infinite
-// and NaN bounds included) are computed in f64 as before.  Per chunk the lanes
-// first compute the candidate with their largest bound, so that already the
-// first chunk of a row leaves one or two f64 evaluations for 512 logits.
-// Bounded by the integer hash (two 64-bit products per logit).
-// 256 x 126464 logits at temperature 1 on an MI355X: 154 -> 42 us.
+// A threshold follows from a value that the row is known to hold: at first from
+// lower bounds over a wavefront's first chunk, then from the largest value that
+// any wavefront of the workgroup has computed (in LDS).  A logit whose bound is
+// below it is left out, all others (infinite and NaN bounds included) are
+// computed in f64 as before, the ones with the lanes' largest bounds first.
+// Bounded by the integer hash (two 64-bit products per logit, six quarter-rate
+// multiplies).  256 x 126464 logits at temperature 1 on an MI355X: 154 us
+// without the bound, 42 us with one logarithm per logit and a threshold per
+// wavefront, 35.6 us now.
 constexpr float kNoiseGap = 110.0f;
 
-// log2 of the bound above for one logit; z1 = seed + (counter + 1) * golden.
-__device__ __forceinline__ float noise_bound_log2(float l, float T, uint64_t z1) {
+// High word of the draw's SplitMix64 product, z1 = seed + (counter + 1) * golden;
+// the generator's last step xors its own top bit into the word's lowest one.
+__device__ __forceinline__ uint32_t noise_high(uint64_t z1) {
   uint64_t z = z1;
   z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
   z ^= z >> 27;
   const uint32_t lo = (uint32_t)z, hi = (uint32_t)(z >> 32);
-  // high word of z * 0x94D049BB133111EB, then of its xor with itself >> 31
-  uint32_t h = __umulhi(lo, 0x133111EBu) + lo * 0x94D049BBu + hi * 0x133111EBu;
-  h ^= h >> 31;
+  return __umulhi(lo, 0x133111EBu) + lo * 0x94D049BBu + hi * 0x133111EBu;  // of z * 0x94D049BB133111EB
+}
+
+// log2 of the bound above for one logit with h = hi.
+__device__ __forceinline__ float noise_bound_log2(float l, float T, uint32_t hi) {
+  const uint32_t h = hi ^ (hi >> 31);
   const float lg = __builtin_amdgcn_logf((float)~h) - 32.0f;  // log2; -inf when ~h is 0
   return __builtin_fmaf(l, kLog2e, -T * lg);
+}
+
+// log2 of a lower bound of the value: E <= -log(h 2^-32) (1e-5 for the rounding
+// of the logarithm near h = 2^32), and half a bf16 step down.
+__device__ __forceinline__ float noise_floor_log2(float l, float T, uint32_t hi) {
+  const uint32_t h = hi ^ (hi >> 31);
+  const float E = 0.69314718f * (32.0f - __builtin_amdgcn_logf((float)h)) + 1e-5f;  // inf when h is 0
+  return __builtin_fmaf(l, kLog2e, -T * __builtin_amdgcn_logf(E)) - (0.01f + 1e-3f * T);
 }
 
 // log2 below which a bound means "kNoiseGap below m_w, or less" (m_w: a value
@@ -178,17 +192,43 @@ __device__ __forceinline__ float wave_max(float x) {
 // Fold 8 logits of a row with temperature T into (m, s, i); rc + e0 = counter
 // of the first.  thr: the wavefront's threshold.  All 64 lanes call it; those
 // with `live` false hold no logits.
-__device__ __forceinline__ void smx_noisy_chunk(u32x4_t v, int e0, bool live, double T, uint64_t seed, uint64_t rc,
-                                                float& m, float& s, int& i, float& thr) {
+__device__ __forceinline__ void smx_noisy_chunk(u32x4_t v, int e0, bool live, double T, float inv_T, uint64_t seed,
+                                                uint64_t rc, float& m, float& s, int& i, float& thr,
+                                                uint32_t* best) {
   float f[8], b[8];
+  uint32_t hi[8];
   smx_unpack(v, f);
   const float Tf = (float)T;
+  // One limit for the chunk: a logit up to its largest one has a bound below thr
+  // unless log2(2^32 - 1 - h) <= 32 + (lmax log2(e) - thr) / T, so that each
+  // logit costs its hash and one comparison (a NaN logit makes the maximum, and
+  // with it the limit, NaN: everything passes).
+  float lmax = f[0];
+#pragma unroll
+  for (int k = 1; k < 8; ++k) lmax = __builtin_elementwise_maximum(lmax, f[k]);
+  const float x = __builtin_amdgcn_exp2f(32.0f + (lmax * kLog2e - thr) * inv_T);
+  // thr's slack covers the rounding of the difference, the factor that of the sum
+  // and of exp2; two more for the xored bit and the conversion
+  const uint32_t lim = x < 4.2e9f ? (uint32_t)(x * 1.002f) + 2u : 0xffffffffu;
   uint64_t z = seed + (rc + (uint64_t)e0 + 1) * 0x9E3779B97F4A7C15ull;
+  bool any = false;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    hi[k] = noise_high(z);
+    z += 0x9E3779B97F4A7C15ull;
+    any |= ~hi[k] <= lim;
+  }
+  if (!__builtin_amdgcn_ballot_w64(live && any)) return;
+  if (thr == -INFINITY) {  // the wavefront knows no value yet
+    float lb = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) lb = fmaxf(lb, noise_floor_log2(f[k], Tf, hi[k]));
+    thr = noise_threshold(__builtin_amdgcn_exp2f(fminf(wave_max(live ? lb : -INFINITY), 126.0f)), Tf);
+  }
   uint32_t pend = 0;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    b[k] = noise_bound_log2(f[k], Tf, z);
-    z += 0x9E3779B97F4A7C15ull;
+    b[k] = noise_bound_log2(f[k], Tf, hi[k]);
     pend |= !(b[k] < thr) ? 1u << k : 0u;
   }
   if (!live) pend = 0;
@@ -217,7 +257,9 @@ __device__ __forceinline__ void smx_noisy_chunk(u32x4_t v, int e0, bool live, do
       }
     }
     if (__builtin_amdgcn_ballot_w64(raised)) {
-      thr = fmaxf(thr, noise_threshold(wave_max(m), Tf));
+      const float m_w = wave_max(m);
+      thr = fmaxf(thr, noise_threshold(m_w, Tf));
+      if ((threadIdx.x & 63) == 0 && m_w > 0.f) atomicMax(best, __float_as_uint(m_w));  // ordered like the value
 #pragma unroll
       for (int k = 0; k < 8; ++k) pend &= b[k] < thr ? ~(1u << k) : ~0u;
     }
@@ -279,17 +321,23 @@ __device__ __forceinline__ void smx_scan_noisy(const SmxArgs& a, int row, int c0
   const double T = a.temp[row];
   const uint64_t rc = (uint64_t)(a.row_base + row) * (uint64_t)a.V;
   float thr = -INFINITY;
+  const float inv_T = 1.0f / (float)T;
   const int lead = (int)(threadIdx.x & 63);
-  for (int c = c0 + (int)threadIdx.x; c - lead < c1; c += 4 * NT) {
-    u32x4_t v[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int cc = c + u * NT;
-      v[u] = cc < c1 ? ld128_stream(base + 8 * (int64_t)cc) : ninf;
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      smx_noisy_chunk(v[u], 8 * (c + u * NT), c + u * NT < c1, T, a.seed, rc, m, s, idx, thr);
+  __shared__ uint32_t best;  // the largest value computed, as bits (0: none)
+  if (threadIdx.x == 0) best = 0;
+  __syncthreads();
+  // one chunk at a time, the next one's load in flight: the chunk's code with its
+  // f64 functions is long, and a second copy of it costs instruction fetches
+  auto load = [&](int c) { return c < c1 ? ld128_stream(base + 8 * (int64_t)c) : ninf; };
+  int c = c0 + (int)threadIdx.x;
+  u32x4_t v = load(c);
+#pragma unroll 1
+  for (; c - lead < c1; c += NT) {
+    const u32x4_t next = load(c + NT);
+    const float known = __uint_as_float(*(volatile uint32_t*)&best);
+    if (known > 0.f) thr = fmaxf(thr, noise_threshold(known, (float)T));
+    smx_noisy_chunk(v, 8 * c, c < c1, T, inv_T, a.seed, rc, m, s, idx, thr, &best);
+    v = next;
   }
 }
 
@@ -407,17 +455,16 @@ __global__ __launch_bounds__(256) void smx_merge_kernel(SmxArgs a) {
 // Workgroups per row.  A CU takes in at most ~26 GB a millisecond, ~10 us for a
 // row of 253 KB, so few rows are spread over several CUs; the second launch
 // (~2.5 us) pays for that up to 64 rows, and with noise, whose integer hash
-// keeps a CU busy for 40 us a row, wherever CUs would stay idle.  Measured at
+// keeps a CU busy for 35 us a row, wherever CUs would stay idle.  Measured at
 // 126464 logits per row, one workgroup a row against the split: 8 rows 12.3 /
 // 7.8, 32 12.5 / 8.5, 64 12.3 / 9.8, 96 12.4 / 11.6, 128 12.6 / 12.1 us (not
-// split); with noise 8 rows 42 / 17.5, 64 42 / 21.8, 128 42 / 30.5 us.  A range
-// is at least one chunk per thread.
+// split); with noise 8 rows 35 / 10.9, 64 35 / 19.9, 128 35 / 26.0 us.  A range
+// is at least 512 chunks (noise: 256; twice and four times as many ranges:
+// 20.8 and 21.7 us at 64 rows).
 static int smx_splits(int M, int V, bool noisy) {
-  if (M <= 0 || M > (noisy ? 128 : 64)) return 1;
-  int n = 256 / M;
-  if (n > 8) n = 8;
-  const int most = V / 8 / (noisy ? 1024 : 512);
-  if (n > most) n = most;
+  if (M <= 0) return 1;
+  int n = noisy ? min(32, 256 / M) : M <= 64 ? min(8, 256 / M) : 1;
+  n = min(n, V / 8 / (noisy ? 256 : 512));
   return n < 1 ? 1 : n;
 }
 

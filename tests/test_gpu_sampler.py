@@ -69,7 +69,7 @@ def test_softmax_max_matches_oracle(dev, M, V, sigma, pad):
     (20, 16384, 0.3, 0, 0.0),        # ranges merged by the second launch, rescan on every row
     (3, 8232, 1.0, 8, 0.0),          # 1029 chunks in two ranges, strided
     (64, 126464, 2.0, 0, 0.0),       # the most rows that are split
-    (5, 33288, 2.0, 8, 1.0),         # noisy: four ranges of 4161 chunks
+    (5, 33288, 2.0, 8, 1.0),         # noisy: sixteen ranges of 4161 chunks
     (128, 16392, 2.0, 0, 0.5),       # noisy: the most rows that are split
 ])
 def test_softmax_max_split_rows(dev, M, V, sigma, pad, T):

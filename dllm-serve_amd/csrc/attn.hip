@@ -1385,11 +1385,12 @@ static DensePlan dense_plan(int n_seg, int max_seqlen_q, int max_seqlen_k, int H
   // 9.1 / 9.0, 8.2, 8.0; 1 x 512 13.7 / 13.0, 11.8, 12.7; 1 x 640 16.2 / 15.3,
   // 19.3, 16.3; 4 x 256 10.5 / 10.2, 12.4, 11.6.  Four wavefronts up to three
   // workgroups on two CUs: 1 x 1280 (320 workgroups) 40.0 / 38.5, 4 x 384 (384)
-  // 19.1 / 19.0, 8 x 384 as 768 29 / 30 (not taken).
+  // 19.6 / 19.4, 8 x 384 as 768 29 / 30 (not taken); and from 192 keys on: 4 x
+  // 139 tokens 7.8 / 7.9, 6 x 139 10.95 / 11.1, 4 x 200 9.4 / 9.15.
   if (!wide) {
     const int64_t pairs = (int64_t)n_seg * Hkv;
     auto groups = [&](int nw) { return pairs * ((m_rows + 32 * nw - 1) / (32 * nw)); };
-    const int nw = groups(1) <= 256 ? 1 : groups(2) <= 256 ? 2 : groups(4) <= 384 ? 4 : 0;
+    const int nw = groups(1) <= 256 ? 1 : groups(2) <= 256 ? 2 : max_seqlen_k >= 192 && groups(4) <= 384 ? 4 : 0;
     p.piped = nw > 0;
     if (nw) p.nw = nw;
   }

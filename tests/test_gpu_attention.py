@@ -384,8 +384,8 @@ def test_block_cached_invalid_slots_are_excluded(dev, Hq, Hkv):
     (28, 4, 9, 97, 1),       # grouped heads, rows past the segment in the row block
     (32, 32, 257, 95, 2),    # 9 row blocks of 32 per head: 288 workgroups of one
     (32, 32, 512, 512, 2),
-    (32, 32, 513, 160, 4),
-    (28, 4, 800, 129, 4),
+    (32, 32, 513, 200, 4),
+    (28, 4, 800, 193, 4),
     (4, 4, 40, 0, 1),        # no keys: zero rows
 ])
 def test_piped_launch_rows_equal_a_batch(dev, Hq, Hkv, lq, lk, wavefronts):

@@ -565,7 +565,31 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC, OC
       __syncthreads();
       ot = lds + wave * 8192;
     }
-    store_o_rows(a, ot, st.oacc[0], inv, qrow0, hkv, m_base + wave * 32, M, lane);
+    // store_o_rows' steps, kept inline: as a call of it the compiler orders the
+    // whole kernel differently (8 x 384 tokens, 32 heads: 28.98 us in alternating
+    // runs, 28.95 inline)
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int rq = 0; rq < 4; ++rq) {
+        u32x2_t w;
+        w[0] = cvt_pk_bf16(st.oacc[0][db][4 * rq + 0] * inv, st.oacc[0][db][4 * rq + 1] * inv);
+        w[1] = cvt_pk_bf16(st.oacc[0][db][4 * rq + 2] * inv, st.oacc[0][db][4 * rq + 3] * inv);
+        const int chunk = 4 * db + rq;
+        *reinterpret_cast<u32x2_t*>(ot + lrow * 256 + ((chunk ^ (lrow & 15)) * 16) + 8 * hl) = w;
+      }
+    const int rsub = lane >> 4, ch = lane & 15;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int r = 4 * j + rsub;
+      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ot + r * 256 + ((ch ^ (r & 15)) * 16));
+      const int m = m_base + wave * 32 + r;
+      if (m < M) {
+        const int tok = m / g;
+        const int head = hkv * g + (m - tok * g);
+        st128(a.o + (int64_t)(qrow0 + tok) * a.o_stride + head * HD + ch * 8, v);
+      }
+    }
   } else {
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {

@@ -53,6 +53,7 @@ struct AttnArgs {
   int logical_blocks;
   int xcd_chunk;      // logical blocks per chunk of the XCD interleave (grid = multiple of 8 * xcd_chunk)
   float scale_log2;
+  int fold_tiles;     // K3b: 128-key tiles of the first of a workgroup's two key splits (0: it has one)
 };
 
 // Work-groups are dispatched round-robin over the 8 XCDs (XCD = b % 8), and
@@ -828,72 +829,36 @@ __device__ __forceinline__ void gdma16(const void* g, uint8_t* lds_dst) {
   __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)lds_dst, 16, 0, kStreamAux);
 }
 
-// The four wavefronts' softmax states of one row block (each holds the same
-// 32 M rows over its own keys) merged, normalised and written to o -- or,
-// when the keys are split across workgroups, written as a partial record
-// for attn_combine_kernel.  Every thread of the workgroup calls it once (it
-// holds workgroup barriers).  The four wavefronts of a row block park their
-// unscaled O^T partials as [row][d] f32 in 32 rows x 2 x 256 bytes of a
-// stage (d 0..63 in the K rows, 64..127 in the V rows of their key block;
-// 16-byte chunk c of a row at c ^ (row & 15),
-// so that 16 lanes on 16 rows hit 16 different chunks), and their row maxima
-// and sums in the idle slot ring.  Row block 0 uses the stage the last tile
-// did not use, free once every wavefront has passed the last tile's first
-// barrier (with RB = 1 a wavefront only ever reads its own rows, so at once);
-// row block 1 uses the last tile's stage after one more barrier.  Then thread
-// (row q, d0 .. d0 + 15) of each row block merges its four partials,
-// wavefronts in order, each scaled term (and each term of the row sum)
-// rounded before it is added.
-template <int RB, int DS>
-__device__ __forceinline__ void cached_merge_store(const AttnArgs& a, uint8_t* lds, int last_stage, float* ring,
-                                                        const DenseState<1>& st, int s, int hkv, int mt, int split,
-                                                        int qrow0, int M, int m_base, int g, int tid, int rblk,
-                                                        int dpart) {
-  constexpr int NDB = 4 / DS;     // d blocks of 32 this workgroup owns
-  constexpr int DPT = 16 / DS;    // d positions a thread merges
-  const int dbase = dpart * 32 * NDB;
-  const int wave = (tid >> 6) & 3;
-  const int lane = tid & 63;
-  const int lrow = lane & 31;
-  const int hl = lane >> 5;
-  // piece p of wave w: part + p * CK_TILE * 256 + w * 8 KiB
-  uint8_t* part = lds + (rblk == 0 ? last_stage ^ 1 : last_stage) * CK_STAGE;
-  float* ml = ring + rblk * 4 * 2 * 32;
-  const float l_tot = pair_sum32(st.l_run[0]);
-  if (hl == 0) {
-    ml[(wave * 2 + 0) * 32 + lrow] = st.m_run[0];
-    ml[(wave * 2 + 1) * 32 + lrow] = l_tot;
-  }
-  auto park = [&]() {
+// Parks NDB d blocks of a wavefront's unscaled O^T as [row][d] f32 in its 32 rows
+// of a stage (d 0..63 in the K rows, 64..127 in the V rows; 16-byte chunk c of a
+// row at c ^ (row & 15), so that 16 lanes on 16 rows hit 16 different chunks).
+template <int NDB>
+__device__ __forceinline__ void cached_park(uint8_t* part, const f32x16_t* o, int wave, int lrow, int hl) {
 #pragma unroll
-    for (int db = 0; db < NDB; ++db)
+  for (int db = 0; db < NDB; ++db)
 #pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        const int d = db * 32 + 8 * rq + 4 * hl;
-        uint8_t* row = part + (d >> 6) * CK_TILE * 256 + (wave * 32 + lrow) * 256;
-        const f32x4_t v = {st.oacc[0][db][4 * rq], st.oacc[0][db][4 * rq + 1], st.oacc[0][db][4 * rq + 2],
-                           st.oacc[0][db][4 * rq + 3]};
-        *reinterpret_cast<f32x4_t*>(row + ((((d & 63) >> 2) ^ (lrow & 15)) << 4)) = v;
-      }
-  };
-  if (rblk == 0) park();
-  if constexpr (RB > 1) {
-    lds_barrier();  // every wavefront is done with the last tile's stage
-    if (rblk == 1) park();
-  }
-  lds_barrier();
-  tid &= 255;
-  const int q = tid & 31;
-  const int d0 = (tid >> 5) * DPT;  // inside the workgroup's d range
-  float mw[4], mq = -INFINITY;
+    for (int rq = 0; rq < 4; ++rq) {
+      const int d = db * 32 + 8 * rq + 4 * hl;
+      uint8_t* row = part + (d >> 6) * CK_TILE * 256 + (wave * 32 + lrow) * 256;
+      const f32x4_t v = {o[db][4 * rq], o[db][4 * rq + 1], o[db][4 * rq + 2], o[db][4 * rq + 3]};
+      *reinterpret_cast<f32x4_t*>(row + ((((d & 63) >> 2) ^ (lrow & 15)) << 4)) = v;
+    }
+}
+
+// Row q, DPT positions from d0, of four parked partials merged: the row's
+// maximum, sum and unscaled O.
+template <int DPT>
+__device__ __forceinline__ void cached_merge(const uint8_t* part, const float* ml, int q, int d0, float& mq, float& lq,
+                                             float (&acc)[DPT]) {
+  float mw[4];
+  mq = -INFINITY;
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
     mw[w] = ml[(w * 2) * 32 + q];
     mq = fmaxf(mq, mw[w]);
   }
   const float mq_use = (mq == -INFINITY) ? 0.f : mq;
-  float lq = 0.f;
-  float acc[DPT];
+  lq = 0.f;
 #pragma unroll
   for (int i = 0; i < DPT; ++i) acc[i] = 0.f;
 #pragma unroll
@@ -908,13 +873,21 @@ __device__ __forceinline__ void cached_merge_store(const AttnArgs& a, uint8_t* l
       for (int e = 0; e < 4; ++e) acc[4 * c4 + e] = __fadd_rn(acc[4 * c4 + e], __fmul_rn(v[e], f));
     }
   }
+}
+
+// Row q's merged DPT positions from d (of the whole head) to o, normalised, or
+// to the split's record.  first: this thread also writes the record's row state.
+template <int DPT>
+__device__ __forceinline__ void cached_store(const AttnArgs& a, int s, int hkv, int mt, int split, int qrow0, int M,
+                                             int m_base, int g, int q, int d, bool first, float mq, float lq,
+                                             const float (&acc)[DPT]) {
   const int mrow = m_base + q;
   if (mrow < M) {
     const int tq = mrow / g;
     const int hq = hkv * g + (mrow - tq * g);
     if (a.n_split == 1) {
       const float inv = lq > 0.f ? 1.f / lq : 0.f;
-      uint16_t* op = a.o + (int64_t)(qrow0 + tq) * a.o_stride + hq * HD + dbase + d0;
+      uint16_t* op = a.o + (int64_t)(qrow0 + tq) * a.o_stride + hq * HD + d;
       uint32_t w[DPT / 2];
 #pragma unroll
       for (int i = 0; i < DPT / 2; ++i) w[i] = cvt_pk_bf16(acc[2 * i] * inv, acc[2 * i + 1] * inv);
@@ -927,13 +900,13 @@ __device__ __forceinline__ void cached_merge_store(const AttnArgs& a, uint8_t* l
       }
     } else {
       const int64_t Prec = (((int64_t)s * a.Hkv + hkv) * a.mtiles + mt) * a.n_split + split;
-      float* po = a.ws + (Prec * 32 + q) * HD + dbase + d0;
+      float* po = a.ws + (Prec * 32 + q) * HD + d;
 #pragma unroll
       for (int i = 0; i < DPT; i += 4) {
         f32x4_t v4 = {acc[i], acc[i + 1], acc[i + 2], acc[i + 3]};
         *reinterpret_cast<f32x4_t*>(po + i) = v4;
       }
-      if (d0 == 0 && dpart == 0) {  // one writer per row
+      if (first) {  // one writer per row
         const int64_t nrec = (int64_t)a.n_seg * a.Hkv * a.mtiles * a.n_split;
         float* pml = a.ws + nrec * 32 * HD + (Prec * 32 + q) * 2;
         pml[0] = mq;
@@ -941,6 +914,104 @@ __device__ __forceinline__ void cached_merge_store(const AttnArgs& a, uint8_t* l
       }
     }
   }
+}
+
+// The four wavefronts' softmax states of one row block (each holds the same
+// 32 M rows over its own keys) merged, normalised and written to o -- or,
+// when the keys are split across workgroups, written as a partial record
+// for attn_combine_kernel.  Every thread of the workgroup calls it once (it
+// holds workgroup barriers).  The four wavefronts of a row block park their
+// unscaled O^T partials in a stage, and their row maxima and sums in the idle
+// slot ring.  Row block 0 uses the stage the last tile
+// did not use, free once every wavefront has passed the last tile's first
+// barrier (with RB = 1 a wavefront only ever reads its own rows, so at once);
+// row block 1 uses the last tile's stage after one more barrier.  Then thread
+// (row q, d0 .. d0 + 15) of each row block merges its four partials,
+// wavefronts in order, each scaled term (and each term of the row sum)
+// rounded before it is added.
+template <int RB>
+__device__ __forceinline__ void cached_merge_store(const AttnArgs& a, uint8_t* lds, int last_stage, float* ring,
+                                                        const DenseState<1>& st, int s, int hkv, int mt, int split,
+                                                        int qrow0, int M, int m_base, int g, int tid, int rblk) {
+  const int wave = (tid >> 6) & 3;
+  const int lane = tid & 63;
+  const int lrow = lane & 31;
+  const int hl = lane >> 5;
+  // piece p of wave w: part + p * CK_TILE * 256 + w * 8 KiB
+  uint8_t* part = lds + (rblk == 0 ? last_stage ^ 1 : last_stage) * CK_STAGE;
+  float* ml = ring + rblk * 4 * 2 * 32;
+  const float l_tot = pair_sum32(st.l_run[0]);
+  if (hl == 0) {
+    ml[(wave * 2 + 0) * 32 + lrow] = st.m_run[0];
+    ml[(wave * 2 + 1) * 32 + lrow] = l_tot;
+  }
+  if (rblk == 0) cached_park<4>(part, st.oacc[0], wave, lrow, hl);
+  if constexpr (RB > 1) {
+    lds_barrier();  // every wavefront is done with the last tile's stage
+    if (rblk == 1) cached_park<4>(part, st.oacc[0], wave, lrow, hl);
+  }
+  lds_barrier();
+  tid &= 255;
+  const int q = tid & 31;
+  const int d0 = (tid >> 5) * 16;
+  float mq, lq, acc[16];
+  cached_merge<16>(part, ml, q, d0, mq, lq, acc);
+  cached_store<16>(a, s, hkv, mt, split, qrow0, M, m_base, g, q, d0, d0 == 0, mq, lq, acc);
+}
+
+// A wavefront's softmax state over a finished key split (NDB d blocks of 32).
+template <int NDB>
+struct CachedPart {
+  f32x16_t o[NDB];
+  float m, l;
+};
+
+// The merge of a workgroup with one of DS head-dim parts (one row block) and, if
+// `two`, with two key splits (`first`: the state of the first): each split's
+// four partials are merged as a split launch merges them, then the splits as
+// attn_combine_kernel does -- the same products, sums and roundings, so the same
+// bits.  A split's partials take 32 KiB of stage 0 and an entry of the ring each;
+// a wavefront writes only rows and words that itself alone has read.
+template <int DS, int NF>
+__device__ __forceinline__ void cached_parts_store(const AttnArgs& a, uint8_t* lds, float* ring,
+                                                   const CachedPart<4 / DS>& first, bool two, const DenseState<1>& st,
+                                                   int s, int hkv, int mt, int split, int qrow0, int M, int m_base, int g,
+                                                   int tid, int dpart) {
+  constexpr int NDB = 4 / DS;   // d blocks of 32 this workgroup owns
+  constexpr int DPT = 16 / DS;  // d positions a thread merges
+  const int wave = tid >> 6;
+  const int lane = tid & 63;
+  const int lrow = lane & 31;
+  const int hl = lane >> 5;
+  uint8_t* const part1 = lds + CK_TILE * 256;
+  float* const ml1 = ring + 256;
+  auto park = [&](const f32x16_t* o, float m, float l, uint8_t* part, float* ml) {
+    const float l_tot = pair_sum32(l);
+    if (hl == 0) {
+      ml[(wave * 2 + 0) * 32 + lrow] = m;
+      ml[(wave * 2 + 1) * 32 + lrow] = l_tot;
+    }
+    cached_park<NDB>(part, o, wave, lrow, hl);
+  };
+  park(st.oacc[0], st.m_run[0], st.l_run[0], lds, ring);
+  if (NF > 1 && two) park(first.o, first.m, first.l, part1, ml1);
+  lds_barrier();
+  const int q = tid & 31;
+  const int d0 = (tid >> 5) * DPT;  // inside the workgroup's d range
+  float mq, lq, acc[DPT];
+  cached_merge<DPT>(lds, ring, q, d0, mq, lq, acc);
+  if (NF > 1 && two) {
+    float m1, l1, acc1[DPT];
+    cached_merge<DPT>(part1, ml1, q, d0, m1, l1, acc1);
+    const float mx = fmaxf(m1, mq), mu = (mx == -INFINITY) ? 0.f : mx;
+    const float w1 = (m1 == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m1 - mu);
+    const float w = (mq == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mq - mu);
+    lq = __builtin_fmaf(lq, w, l1 * w1);
+#pragma unroll
+    for (int i = 0; i < DPT; ++i) acc[i] = __builtin_fmaf(acc[i], w, acc1[i] * w1);
+  }
+  cached_store<DPT>(a, s, hkv, mt, split, qrow0, M, m_base, g, q, dpart * 32 * NDB + d0, d0 == 0 && dpart == 0, mq, lq,
+                    acc);
 }
 
 // One 32-key block of the four-wavefront K3b: K operands from LDS, keys set in
@@ -1011,7 +1082,11 @@ __device__ __forceinline__ void cached_tile(const uint8_t* Ks, const uint8_t* Vs
 // CU takes in 26-50 KB a microsecond however idle the chip is, so a launch of
 // few workgroups is bound by each one's bytes: 1 - (1 - 1 / DS) / 2 of them are
 // left (K again from the L2 they share), without partials to merge.
-template <int RB, bool PAGED, int DS>
+// NF = 2 (with DS > 1): the workgroup computes two key splits in turn, the
+// second from a fresh softmax state; the first one's waits in registers for the
+// merge.  Two loops over the tiles: as a branch inside one loop the change of
+// state cost up to 0.8 us (copies of the state in every turn).
+template <int RB, bool PAGED, int DS, int NF>
 // The launch geometry and the tables the first, dependent loads read come as
 // leading scalar arguments (14 dwords): the library is built with kernel
 // argument preloading, so they are in SGPRs when a wave starts instead of one
@@ -1246,7 +1321,7 @@ __global__ __launch_bounds__(256 * RB) __attribute__((amdgpu_waves_per_eu(2, 2))
   dense_state_init(st);
   const float c = a.scale_log2;
 
-  for (int t = 0; t < ntiles; ++t) {
+  auto tile_turn = [&](int t) {
     const int k0 = kbeg + t * CK_TILE;
     // D(t) has landed once at most the operations issued after it -- S(t+2)
     // and D(t+1), when they exist -- are outstanding.  At t = 0 only D(1)
@@ -1277,9 +1352,29 @@ __global__ __launch_bounds__(256 * RB) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
     bad_t0 = bad_t1;
     bad_t1 = bad_t2;
+  };
+  CachedPart<4 / DS> first;  // NF > 1: the state of the first key split
+  const int n_first = NF > 1 ? min(a.fold_tiles, ntiles) : ntiles;
+  const bool two = ntiles > n_first;
+  int t = 0;
+#pragma unroll 1
+  for (int f = 0; f < NF; ++f) {
+    const int t_end = f == 0 ? n_first : ntiles;
+    for (; t < t_end; ++t) tile_turn(t);
+    if (NF > 1 && f == 0) {
+#pragma unroll
+      for (int db = 0; db < 4 / DS; ++db) first.o[db] = st.oacc[0][db];
+      first.m = st.m_run[0];
+      first.l = st.l_run[0];
+      if (two) dense_state_init(st);
+    }
   }
-  cached_merge_store<RB, DS>(a, lds, (ntiles - 1) & 1, reinterpret_cast<float*>(slot_ring), st, s, hkv, mt, split,
-                             qrow0, M, m_base, g, tid, rblk, dpart);
+  if constexpr (DS > 1)
+    cached_parts_store<DS, NF>(a, lds, reinterpret_cast<float*>(slot_ring), first, two, st, s, hkv, mt, split, qrow0, M,
+                               m_base, g, tid, dpart);
+  else
+    cached_merge_store<RB>(a, lds, (ntiles - 1) & 1, reinterpret_cast<float*>(slot_ring), st, s, hkv, mt, split, qrow0,
+                           M, m_base, g, tid, rblk);
 }
 
 // Merge the n_split partial records of every (segment, head, M row).
@@ -1501,58 +1596,68 @@ extern "C" int dllm_attn_varlen_fwd(const dllm_bf16* q, const dllm_bf16* k, cons
 // against 732 keys: 448 -> 256 workgroups, 28 -> 19.5 us); otherwise 1,
 // which streams the same bytes with twice the workgroups (4 x 32 heads x 2 M
 // tiles against 672 keys: 16.5 us, against 19.3 us paired on 128 CUs).
-// Then the keys of more than six 128-key tiles are split, only while the splits
-// still fit in one generation and with at least three tiles each: the partial
-// records and the combine launch cost about 4 us, three tiles of a workgroup's
-// stream.  Measured unsplit / split in us: 384 keys, 1 x 32 rows x 32 heads 9.6
-// / 11.9, 4 x 32 10.6 / 15.1; 672 keys, 2 x 64 14.4 / 15.6; 732 keys, 28 / 4
-// heads, 4 x 32 13.4 / 14.8; 1032 keys, 1 x 32, 28 / 4 16.5 / 13.9 (three
-// tiles a split; two 14.2); 1532 keys, 32 heads 22.5 / 16.1 (two tiles 16.7).
-// Fewer splits cost some accuracy: the relative error against 64 bits is 2-5 %
-// larger than with splits of two tiles (1 x 32 rows against 352, 32 heads
-// 0.002130 -> 0.002231), as large as that of launches never split.
-// Up to 32 workgroups gain from six tiles on: 732 keys, 1 x 32 rows x 32 heads
-// 13.8 / 13.4 (three splits of two tiles).
+// Then the keys are split while the splits still fit in one generation, with at
+// least two 128-key tiles each.  A split rounds its probabilities to bf16
+// against its own maxima (the largest of a row then rounds to exactly 1), so
+// fewer splits are a little less accurate -- 1 x 32 rows against 352, 32 heads:
+// relative error against 64 bits 0.002148 with two, 0.002246 with one -- and the
+// number of splits is not lowered for speed.  Two splits of up to six tiles in all are
+// computed by one workgroup in turn (fold_tiles; the same bits): the partial
+// records and the combine launch of two workgroups cost more (~4 us).  Measured
+// two workgroups / one, in us: 384 keys, 1 x 32 rows x 32 heads 10.4 / 8.7, 4 x 32
+// 15.1 / 10.6; 640 keys, 4 x 32 17.7 / 14.3; 732 keys, 28 / 4 heads, 4 x 32 14.5 /
+// 13.8; 1032 keys (nine tiles) 16.8 / 18.1.  Three splits in turn gain nothing:
+// 532 keys, 1 x 32 rows x 32 heads 11.7 / 12.4, 640 keys, 1 x 64 13.9 / 14.0.
 // Launches that still leave CUs idle deal the output's d positions to 2 or 4
 // workgroups, as many as one generation holds.  Measured with 1 / 2 / 4 in us,
 // caches from HBM: 1 x 32 rows x 32 heads against 352 cached rows 10.1 / 8.9 /
 // 8.4, 2 x 32 10.5 / 9.4 / 8.9, 4 x 32 (128 workgroups) 11.1 / 10.2 / 16.5; 1 x
 // 64 against 608 14.2 / 13.0 / 12.5; 28 / 4 heads, 4 x 32 against 700 13.8 / 12.8
-// / 23.2; 1 x 32 against 1500 (four key splits) 15.9 / 14.6 / 20.8.
-static int block_cached_plan(int n_seg, int max_q, int max_keys, int Hq, int Hkv, int& mtiles, int& rb,
-                             int& n_split, int& keys_per_split, int& d_split) {
+// / 23.2 (each with one key split).
+struct CachedPlan {
+  int mtiles, rb;               // row blocks of 32 M rows, and of a workgroup
+  int n_split, keys_per_split;  // workgroups along the keys, and the keys of each
+  int fold_tiles;               // 128-key tiles of the first of a workgroup's two key splits (0: it has one)
+  int d_split;                  // workgroups along the head dim
+};
+static CachedPlan block_cached_plan(int n_seg, int max_q, int max_keys, int Hq, int Hkv) {
   const int g = Hq / Hkv;
-  mtiles = (max_q * g + 31) / 32;
-  const int64_t pairs1 = (int64_t)n_seg * Hkv * mtiles;
-  const int64_t pairs2 = (int64_t)n_seg * Hkv * ((mtiles + 1) / 2);
-  rb = (mtiles >= 2 && (pairs1 + 255) / 256 > (pairs2 + 255) / 256) ? 2 : 1;
-  const int64_t pairs = rb == 2 ? pairs2 : pairs1;
+  CachedPlan p = {};
+  p.mtiles = (max_q * g + 31) / 32;
+  const int64_t pairs1 = (int64_t)n_seg * Hkv * p.mtiles;
+  const int64_t pairs2 = (int64_t)n_seg * Hkv * ((p.mtiles + 1) / 2);
+  p.rb = (p.mtiles >= 2 && (pairs1 + 255) / 256 > (pairs2 + 255) / 256) ? 2 : 1;
+  const int64_t pairs = p.rb == 2 ? pairs2 : pairs1;
   int64_t want = pairs > 0 ? 256 / pairs : 1;
-  const int tiles = (max_keys + CK_TILE - 1) / CK_TILE;
-  const int max_split = pairs <= 32 && tiles >= 6 ? (tiles < 9 ? 3 : tiles / 3) : tiles > 6 ? tiles / 3 : 1;
+  const int max_split = max_keys > 0 ? (max_keys + 255) / 256 : 1;
   if (want > max_split) want = max_split;
   if (want < 1) want = 1;
-  n_split = (int)want;
-  const int tiles_per_split = (tiles + n_split - 1) / n_split;
-  keys_per_split = tiles_per_split * CK_TILE;
-  if (keys_per_split <= 0) keys_per_split = CK_TILE;
-  // a split's keys span at most 64 pages of 256 rows: the page-table form
-  // keeps that many page ids per wavefront in LDS (both forms plan alike, so
+  p.n_split = (int)want;
+  const int tiles = (max_keys + CK_TILE - 1) / CK_TILE;
+  const int tiles_per_split = (tiles + p.n_split - 1) / p.n_split;
+  p.keys_per_split = tiles_per_split * CK_TILE;
+  if (p.keys_per_split <= 0) p.keys_per_split = CK_TILE;
+  // a split's keys touch at most 64 of the page-table form's 256-row pages,
+  // so one wavefront's page ids stay in one register (both forms split alike:
   // one workspace size serves both)
-  if (keys_per_split > 64 * 256 - 256) keys_per_split = 64 * 256 - 256;
-  n_split = max_keys > 0 ? (max_keys + keys_per_split - 1) / keys_per_split : 1;
-  const int64_t groups = pairs * n_split;
-  d_split = rb > 1 ? 1 : groups * 4 <= 256 ? 4 : groups * 2 <= 256 ? 2 : 1;
-  return 0;
+  if (p.keys_per_split > 64 * 256 - 256) p.keys_per_split = 64 * 256 - 256;
+  p.n_split = max_keys > 0 ? (max_keys + p.keys_per_split - 1) / p.keys_per_split : 1;
+  if (p.n_split == 2 && p.rb == 1 && pairs <= 128 && tiles <= 6) {
+    p.fold_tiles = p.keys_per_split / CK_TILE;
+    p.keys_per_split *= p.n_split;
+    p.n_split = 1;
+  }
+  const int64_t groups = pairs * p.n_split;
+  p.d_split = p.rb > 1 ? 1 : groups * 4 <= 256 ? 4 : groups * 2 <= 256 ? 2 : 1;
+  return p;
 }
 
 extern "C" size_t dllm_attn_block_cached_workspace_size(int n_seg, int max_q, int max_keys, int Hq, int Hkv, int D) {
   (void)D;
   if (n_seg <= 0 || max_q <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv) return 0;
-  int mtiles, rb, n_split, kps, ds;
-  block_cached_plan(n_seg, max_q, max_keys, Hq, Hkv, mtiles, rb, n_split, kps, ds);
-  if (n_split <= 1) return 0;
-  const size_t nrec = (size_t)n_seg * Hkv * mtiles * n_split;
+  const CachedPlan p = block_cached_plan(n_seg, max_q, max_keys, Hq, Hkv);
+  if (p.n_split <= 1) return 0;
+  const size_t nrec = (size_t)n_seg * Hkv * p.mtiles * p.n_split;
   return nrec * 32 * (HD + 2) * sizeof(float);
 }
 
@@ -1560,9 +1665,9 @@ extern "C" int dllm_attn_block_cached_launch_shape(int n_seg, int max_q, int max
                                                    int* row_blocks, int* n_split, int* grid) {
   if (D != HD || Hq <= 0 || Hkv <= 0 || Hq % Hkv || n_seg < 0 || max_q < 0 || max_keys < 0)
     return fail(DLLM_ERR_INVALID_ARG, "dllm_attn_block_cached_launch_shape: unsupported sizes");
-  int mtiles = 0, rb = 1, ns = 1, kps = 0, ds = 1;
-  block_cached_plan(n_seg, max_q, max_keys, Hq, Hkv, mtiles, rb, ns, kps, ds);
-  const int mblocks = (mtiles + rb - 1) / rb;
+  const CachedPlan p = block_cached_plan(n_seg, max_q, max_keys, Hq, Hkv);
+  const int rb = p.rb, ns = p.n_split, ds = p.d_split;
+  const int mblocks = (p.mtiles + rb - 1) / rb;
   const int64_t logical = (int64_t)ds * ns * mblocks * Hkv * n_seg;
   const int64_t per_pair = (int64_t)ds * ns * mblocks;
   const int64_t grain = 8 * (per_pair < 16 ? per_pair : 16);
@@ -1609,9 +1714,10 @@ static int block_cached_impl(const char* name, const dllm_bf16* q, const dllm_bf
   a.cu_q = cu; a.cu_k = cu; a.seg_ids = seg_ids; a.slots = slots; a.slot_off = slot_off;
   a.q_stride = q_stride_tok; a.k_stride = k_stride_tok; a.v_stride = v_stride_tok; a.o_stride = o_stride_tok;
   a.n_seg = n_seg; a.Hkv = Hkv; a.g = Hq / Hkv;
-  int mtiles, rb, n_split, kps, ds;
-  block_cached_plan(n_seg, max_q, max_keys, Hq, Hkv, mtiles, rb, n_split, kps, ds);
-  a.mtiles = mtiles; a.n_split = n_split; a.keys_per_split = kps;
+  const CachedPlan p = block_cached_plan(n_seg, max_q, max_keys, Hq, Hkv);
+  const int mtiles = p.mtiles, rb = p.rb, n_split = p.n_split, ds = p.d_split;
+  a.mtiles = mtiles; a.n_split = n_split; a.keys_per_split = p.keys_per_split;
+  a.fold_tiles = p.fold_tiles;
   if (n_split > 1) {
     const size_t need = dllm_attn_block_cached_workspace_size(n_seg, max_q, max_keys, Hq, Hkv, D);
     if (!workspace || workspace_bytes < need)
@@ -1647,13 +1753,17 @@ static int block_cached_impl(const char* name, const dllm_bf16* q, const dllm_bf
     return paged ? launch(page_form, threads, lds_bytes) : launch(slot_form, threads, lds_bytes);
   };
   if (rb == 2)
-    rc = pick(attn_cached_kernel<2, false, 1>, attn_cached_kernel<2, true, 1>, 512, ck_lds_bytes(2));
+    rc = pick(attn_cached_kernel<2, false, 1, 1>, attn_cached_kernel<2, true, 1, 1>, 512, ck_lds_bytes(2));
+  else if (ds == 4 && p.fold_tiles)
+    rc = pick(attn_cached_kernel<1, false, 4, 2>, attn_cached_kernel<1, true, 4, 2>, 256, ck_lds_bytes(1));
   else if (ds == 4)
-    rc = pick(attn_cached_kernel<1, false, 4>, attn_cached_kernel<1, true, 4>, 256, ck_lds_bytes(1));
+    rc = pick(attn_cached_kernel<1, false, 4, 1>, attn_cached_kernel<1, true, 4, 1>, 256, ck_lds_bytes(1));
+  else if (p.fold_tiles)
+    rc = pick(attn_cached_kernel<1, false, 2, 2>, attn_cached_kernel<1, true, 2, 2>, 256, ck_lds_bytes(1));
   else if (ds == 2)
-    rc = pick(attn_cached_kernel<1, false, 2>, attn_cached_kernel<1, true, 2>, 256, ck_lds_bytes(1));
+    rc = pick(attn_cached_kernel<1, false, 2, 1>, attn_cached_kernel<1, true, 2, 1>, 256, ck_lds_bytes(1));
   else
-    rc = pick(attn_cached_kernel<1, false, 1>, attn_cached_kernel<1, true, 1>, 256, ck_lds_bytes(1));
+    rc = pick(attn_cached_kernel<1, false, 1, 1>, attn_cached_kernel<1, true, 1, 1>, 256, ck_lds_bytes(1));
   if (rc) return rc;
   if ((rc = check_launch(name))) return rc;
   if (n_split > 1) {

@@ -422,12 +422,12 @@ def test_piped_launch_rows_equal_a_batch(dev, Hq, Hkv, lq, lk, wavefronts):
 
 @pytest.mark.parametrize("paged", [False, True])
 @pytest.mark.parametrize("n_seg,Hq,Hkv,lq,nc,parts", [
-    (1, 32, 32, 32, 352, 4),     # 32 workgroups: four per (segment, KV head), 32 d positions each
+    (1, 32, 32, 32, 224, 4),     # 32 workgroups: four per (segment, KV head), 32 d positions each
     (1, 4, 4, 1, 0, 4),          # one block row, nothing cached
     (2, 28, 4, 9, 129, 4),       # 63 M rows: a row block with one idle row
-    (3, 32, 32, 20, 257, 2),     # 96 workgroups: two
+    (3, 32, 32, 20, 230, 2),     # 96 workgroups: two
     (1, 32, 32, 97, 31, 2),      # four row blocks
-    (4, 32, 32, 32, 608, 2),     # 128 workgroups
+    (4, 32, 32, 32, 97, 2),      # 128 workgroups
 ])
 def test_block_cached_d_parts_equal_a_batch(dev, paged, n_seg, Hq, Hkv, lq, nc, parts):
     """Launches of few workgroups deal the head dim to several of them: the
@@ -478,3 +478,73 @@ def test_block_cached_d_parts_equal_a_batch(dev, paged, n_seg, Hq, Hkv, lq, nc, 
         ref = oatt.block_cached(to_np(q[sl]), to_np(k[sl]), to_np(v[sl]), kcn, vcn, slots[s].tolist(), D ** -0.5,
                                 dtype=np.float32)
         assert_attn_close(alone[sl], ref, f"segment {s}")
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,lq,cached,reach", [
+    (32, 32, 32, [352], 1100),             # three tiles in splits of two and one, four d parts
+    (4, 4, 1, [256], 1100),                # the second split: the block row alone
+    (28, 4, 9, [400, 0, 249, 247], 1100),  # ragged: second splits of 153, 0, 2 and 0 keys
+    (32, 32, 20, [260, 492, 31], 1100),    # 96 workgroups: two d parts
+    (32, 32, 32, [608, 384, 353, 700], 2560),  # six tiles, three to a split
+])
+def test_block_cached_two_splits_in_one_workgroup(dev, paged, Hq, Hkv, lq, cached, reach):
+    """Two key splits computed by one workgroup in turn: bit-equal to the same
+    splits as workgroups of their own -- each segment alone, with a key bound
+    (`reach`) large enough for those -- and more accurate than one split."""
+    print(f"block_cached two splits {Hq}/{Hkv} lq={lq} cached={cached} paged={paged}", flush=True)
+    D, n = 128, len(cached)
+    pages = [-(-c // 256) + 1 for c in cached]
+    g = torch.Generator(device=dev).manual_seed(lq + sum(cached))
+    q = torch.randn(n * lq, Hq, D, generator=g, device=dev).bfloat16()
+    k, v = (torch.randn(n * lq, Hkv, D, generator=g, device=dev).bfloat16() for _ in range(2))
+    kc, vc = (torch.randn(sum(pages) * 256, Hkv, D, generator=g, device=dev).bfloat16() for _ in range(2))
+    ids = torch.randperm(sum(pages), generator=torch.Generator().manual_seed(3)).split(pages)
+    slots = [(i.repeat_interleave(256) * 256 + torch.arange(256).repeat(len(i)))[:c] for i, c in zip(ids, cached)]
+
+    def run(segs, max_keys):
+        x = [torch.cat([t[s * lq:(s + 1) * lq] for s in segs]) for t in (q, k, v)]
+        m = len(segs)
+        cu = (torch.arange(m + 1, device=dev) * lq).int()
+        o = torch.full_like(x[0], float("nan"))
+        ws = torch.empty(max(_capi.block_cached_workspace_size(m, lq, max_keys, Hq, Hkv, D), 16), dtype=torch.uint8,
+                         device=dev)
+        if paged:
+            table = torch.nn.utils.rnn.pad_sequence([ids[s] for s in segs], batch_first=True)
+            _capi.attn_block_cached_paged_fwd(*x, o, cu, None, m, lq, max_keys, kc, vc,
+                                              table.int().contiguous().to(dev),
+                                              torch.tensor([cached[s] for s in segs], dtype=torch.int32, device=dev),
+                                              D ** -0.5, ws)
+        else:
+            off = torch.tensor([0] + [cached[s] for s in segs]).cumsum(0).int().to(dev)
+            _capi.attn_block_cached_fwd(*x, o, cu, None, m, lq, max_keys, kc, vc,
+                                        torch.cat([slots[s] for s in segs] + [torch.zeros(1)]).int().to(dev), off,
+                                        D ** -0.5, ws)
+        torch.cuda.synchronize()
+        return o
+
+    keys = max(cached) + lq
+    assert _capi.block_cached_launch_shape(n, lq, keys, Hq, Hkv, D)["n_split"] == 1
+    assert _capi.block_cached_launch_shape(1, lq, reach, Hq, Hkv, D)["n_split"] > 2
+    o = run(range(n), keys)
+    for s in range(n):
+        alone = run([s], reach)
+        assert torch.equal(o[s * lq:(s + 1) * lq].view(torch.int16), alone.view(torch.int16)), s
+
+    def error(o):
+        num = den = 0.0
+        for s in range(n):
+            ks, vs = (torch.cat([c[slots[s].to(dev)], t[s * lq:(s + 1) * lq]]).double() for c, t in ((kc, k), (vc, v)))
+            for h in range(Hq):
+                w = torch.softmax(q[s * lq:(s + 1) * lq, h].double() @ ks[:, h // (Hq // Hkv)].t().contiguous()
+                                  * D ** -0.5, -1)
+                e = w @ vs[:, h // (Hq // Hkv)].contiguous()
+                num += float((o[s * lq:(s + 1) * lq, h].double() - e).square().sum())
+                den += float(e.square().sum())
+        return (num / den) ** 0.5
+
+    if n * lq * Hq >= 1024:  # enough rows for the errors to differ by less than their 2-5 %
+        copies = -(-160 // (n * Hkv))  # a batch that fills the chip: one split
+        assert _capi.block_cached_launch_shape(n * copies, lq, keys, Hq, Hkv, D)["n_split"] == 1
+        batch = run(list(range(n)) * copies, keys)[:n * lq]
+        assert not torch.equal(batch, o) and error(o) < error(batch) * 0.995

@@ -7,8 +7,10 @@
 // kernels take 9 and 3 us; these forms take 7 and 5 (the step of one 384-token
 // request over 32 layers: 1027 -> 597 us, then bound by the kernels).  Every function here takes the ordinary case only
 // and returns None for anything else -- another type, layout, device or tensor
-// class, and any error of the C ABI -- and the Python form, which raises what
-// is to be raised, runs then.  Nothing is kept between calls.
+// class, and what the C ABI refuses before it launches anything -- and the Python
+// form, which raises what is to be raised, runs then.  A failure of the HIP
+// runtime raises here: the launch may be on the stream already, and a second run
+// would rotate in place, or unmask, twice.  Nothing is kept between calls.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -63,6 +65,12 @@ PyObject* guarded(F f) {
   }
 }
 
+// What a call returns for a code other than DLLM_OK.
+PyObject* refused(const char* what, int rc) {
+  if (rc == DLLM_ERR_INVALID_ARG || rc == DLLM_ERR_UNSUPPORTED || rc == DLLM_ERR_WORKSPACE) Py_RETURN_NONE;
+  return PyErr_Format(PyExc_RuntimeError, "%s failed (code %d): %s", what, rc, dllm_last_error());
+}
+
 // attn(q, k, v, k_cache, v_cache, plan: bytes, scale) -> output or None.
 // `plan` is the packed launch description of one step and head shape.
 struct PlanArgs {
@@ -98,23 +106,26 @@ PyObject* attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const float scale = (float)PyFloat_AS_DOUBLE(a[6]);
     void* st = stream_of((int)p.device);
     auto dev_i32 = [](int64_t x) { return reinterpret_cast<const int32_t*>(x); };
+    const char* what = "dllm_attn_varlen_fwd";
     const int rc = no_gil([&] {
-      int r = 0;
+      int r = DLLM_OK;
       if (p.n_dense)
         r = dllm_attn_varlen_fwd(ptr<dllm_bf16>(*q), ptr<dllm_bf16>(*k), ptr<dllm_bf16>(*v), ptr<dllm_bf16>(o),
                                  dev_i32(p.cu), dev_i32(p.cu), dev_i32(p.dense_ids), (int)p.n_dense,
                                  (int)p.max_q_dense, (int)p.max_q_dense, (int)p.Hq, (int)p.Hkv, (int)p.D, q->stride(0),
                                  k->stride(0), v->stride(0), o.stride(0), scale, st);
-      if (r == 0 && p.n_cached)
+      if (r == DLLM_OK && p.n_cached) {
+        what = "dllm_attn_block_cached_fwd";
         r = dllm_attn_block_cached_fwd(ptr<dllm_bf16>(*q), ptr<dllm_bf16>(*k), ptr<dllm_bf16>(*v), ptr<dllm_bf16>(o),
                                        dev_i32(p.cu), dev_i32(p.cached_ids), (int)p.n_cached, (int)p.max_q_cached,
                                        (int)p.max_keys_cached, ptr<dllm_bf16>(*kc), ptr<dllm_bf16>(*vc), cache_slots,
                                        dev_i32(p.slots), dev_i32(p.slot_off), (int)p.Hq, (int)p.Hkv, (int)p.D,
                                        q->stride(0), k->stride(0), v->stride(0), o.stride(0), scale,
                                        reinterpret_cast<void*>(p.ws), (size_t)p.ws_bytes, st);
+      }
       return r;
     });
-    if (rc != 0) Py_RETURN_NONE;
+    if (rc != DLLM_OK) return refused(what, rc);
     return THPVariable_Wrap(o.dim() == 2 ? std::move(o) : o.view({-1, p.Hq * p.D}));
   });
 }
@@ -152,7 +163,7 @@ PyObject* rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
                             k->stride(0), ptr<dllm_bf16>(ko), ko.stride(0), ptr<int64_t>(*pos), ptr<float>(*cs),
                             cs->size(0), (int)rows, (int)heads[0], (int)heads[1], (int)D, st);
     });
-    if (rc != 0) Py_RETURN_NONE;
+    if (rc != DLLM_OK) return refused("dllm_rope_neox", rc);
     PyObject* x = inplace ? Py_NewRef(a[1]) : THPVariable_Wrap(std::move(qo));
     PyObject* y = inplace ? Py_NewRef(a[2]) : THPVariable_Wrap(std::move(ko));
     PyObject* r = x && y ? PyTuple_Pack(2, x, y) : nullptr;
@@ -181,7 +192,7 @@ PyObject* softmax_max(PyObject*, PyObject* const* a, Py_ssize_t n) {
       return dllm_softmax_max(ptr<dllm_bf16>(*l), l->stride(0), M, V, ptr<int64_t>(x0), ptr<dllm_bf16>(xp),
                               nb ? ws.data_ptr() : nullptr, nb, st);
     });
-    if (rc != 0) Py_RETURN_NONE;
+    if (rc != DLLM_OK) return refused("dllm_softmax_max", rc);
     PyObject* x = THPVariable_Wrap(std::move(x0));
     PyObject* y = THPVariable_Wrap(std::move(xp));
     PyObject* r = x && y ? PyTuple_Pack(2, x, y) : nullptr;
@@ -215,7 +226,7 @@ PyObject* unmask(PyObject*, PyObject* const* a, Py_ssize_t n) {
       return dllm_lowconf_unmask(ptr<int64_t>(*tok), tok->numel(), ptr<int32_t>(*prm), n_seq, (int)win,
                                  ptr<int64_t>(*x0), ptr<dllm_bf16>(*conf), x0->numel(), mask, ptr<int32_t>(out), st);
     });
-    if (rc != 0) Py_RETURN_NONE;
+    if (rc != DLLM_OK) return refused("dllm_lowconf_unmask", rc);
     return THPVariable_Wrap(std::move(out));
   });
 }

@@ -2,6 +2,8 @@
 same calls: the same launches, so bit-equal results, over the layouts both
 take; and what the fast paths leave to the Python forms is still taken or
 refused there."""
+import ctypes
+
 import pytest
 import torch
 
@@ -97,3 +99,60 @@ def test_sampler_calls(dev, both):
     bad = RemaskSampler(lambda h: logits.float(), 9)
     with pytest.raises(ValueError):
         bad.logits_max(torch.empty(48, 8, device=dev))
+
+
+def _pend_hip_error():
+    """Leaves an error of an unrelated host call pending, as any library may:
+    the next check after a launch reports it, with the launch on the stream."""
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64.so" in line)
+    hip = ctypes.CDLL(path)
+    assert hip.hipSetDevice(1 << 20) != 0 and hip.hipPeekAtLastError() != 0
+
+
+def test_runtime_error_after_a_launch_is_raised_once(dev):
+    """A HIP error reported behind a launch raises; the call does not run a
+    second time (rope in place would rotate twice, unmasking go on)."""
+    assert _capi.native is not None, "the native module is not built"
+    rope = RotaryEmbedding(D, D, 64, 10000.0).to(dev)
+    ref = RotaryEmbedding(D, D, 64, 10000.0, inplace=False).to(dev)
+    g = torch.Generator(device=dev).manual_seed(8)
+    q, k = (torch.randn(5, n * D, generator=g, device=dev).bfloat16() for n in (4, 2))
+    pos = torch.arange(5, device=dev)
+    want = ref(pos, q, k)
+    rope.inplace = True
+    torch.cuda.synchronize()
+    _pend_hip_error()
+    with pytest.raises(RuntimeError, match="dllm_rope_neox failed"):
+        rope(pos, q, k)
+    assert torch.equal(q, want[0]) and torch.equal(k, want[1])
+
+    tok = torch.full((1, 16), 9, dtype=torch.int64, device=dev)
+    prm = torch.tensor([[0, 16, 0, 4, 0]], dtype=torch.int32, device=dev)
+    x0 = torch.arange(100, 116, device=dev)
+    conf = torch.rand(16, generator=g, device=dev).bfloat16()
+    logits = torch.randn(16, 64, generator=g, device=dev).bfloat16()
+    torch.cuda.synchronize()
+    _pend_hip_error()
+    with pytest.raises(RuntimeError, match="dllm_lowconf_unmask failed"):
+        # (None would have sample_device_windows unmask a second time)
+        _capi.native.unmask(tok, prm, 16, x0, conf, 9)
+    assert int((tok != 9).sum()) == 4  # ceil(16 / 4): one step
+
+    _pend_hip_error()
+    with pytest.raises(RuntimeError, match="dllm_softmax_max failed"):
+        RemaskSampler(lambda h: logits, 9).logits_max(logits)
+
+    seqs = [Sequence([1] * 24, 8, 9, None, device=dev)]
+    prepare_step(seqs, dev)
+    try:
+        attn = Attention(4, D, D ** -0.5, 4, causal=False)
+        x = torch.randn(32, 4 * D, generator=g, device=dev).bfloat16()
+        attn(x, x, x)
+        torch.cuda.synchronize()
+        _pend_hip_error()
+        with pytest.raises(RuntimeError, match="dllm_attn_varlen_fwd failed"):
+            attn(x, x, x)
+        assert attn(x, x, x).shape == (32, 4 * D)
+    finally:
+        reset_context()

@@ -47,13 +47,15 @@ T* ptr(const at::Tensor& t) {
 
 void* stream_of(int device) { return c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream(); }
 
-// Runs f without the GIL: a launch may wait for a full queue.
+// Runs f without the GIL: a launch may wait for a full queue.  (The GIL is taken
+// back also when f throws: data_ptr() may, where it has to copy first.)
 template <typename F>
 int no_gil(F f) {
-  PyThreadState* s = PyEval_SaveThread();
-  const int rc = f();
-  PyEval_RestoreThread(s);
-  return rc;
+  struct Released {
+    PyThreadState* s = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(s); }
+  } released;
+  return f();
 }
 
 template <typename F>

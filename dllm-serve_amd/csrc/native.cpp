@@ -134,13 +134,14 @@ PyObject* attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // rope(positions, query, key, cos_sin_cache, head_size, inplace) -> (query, key) or None
 PyObject* rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  if (n != 6 || !PyLong_CheckExact(a[4])) Py_RETURN_NONE;
-  const int64_t D = PyLong_AsLongLong(a[4]);
+  if (n != 6 || !PyLong_CheckExact(a[4]) || !PyBool_Check(a[5])) Py_RETURN_NONE;
+  int overflow = 0;
+  const int64_t D = PyLong_AsLongLongAndOverflow(a[4], &overflow);
   const bool inplace = a[5] == Py_True;
   return guarded([&]() -> PyObject* {
     const at::Tensor *pos = plain(a[0], at::kLong), *q = plain(a[1], at::kBFloat16), *k = plain(a[2], at::kBFloat16),
                      *cs = plain(a[3], at::kFloat);
-    if (!pos || !q || !k || !cs || D <= 0 || D > 1024) Py_RETURN_NONE;
+    if (!pos || !q || !k || !cs || overflow || D <= 0 || D > 1024) Py_RETURN_NONE;
     const int dev = q->get_device();
     if (k->get_device() != dev || pos->get_device() != dev || cs->get_device() != dev || pos->dim() != 1 ||
         !pos->is_contiguous() || cs->dim() != 2 || cs->size(1) != D || !cs->is_contiguous())

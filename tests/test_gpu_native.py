@@ -86,6 +86,17 @@ def test_rope_layouts(dev, both, inplace):
             (qa, ka), (qb, kb) = both(call)
             assert qa.shape == qb.shape and qa.stride() == qb.stride()
             assert torch.equal(qa, qb) and torch.equal(ka, kb)
+    # in place is asked for by any true value
+    rope.inplace = int(inplace)
+    (qa, ka), (qb, kb) = both(call)
+    assert torch.equal(qa, qb) and torch.equal(ka, kb)
+    f = fused.clone()
+    rope(pos, f[:, :4 * D], f[:, 4 * D:])
+    assert torch.equal(f, fused) != inplace
+    rope.head_size = 1 << 64  # past every C integer: left to the Python form, which refuses it
+    with pytest.raises((ValueError, TypeError, RuntimeError)):
+        rope(pos, fused[:, :4 * D], fused[:, 4 * D:])
+    rope.head_size = D
     with pytest.raises(ValueError):
         rope(pos, fused.float(), fused)
 

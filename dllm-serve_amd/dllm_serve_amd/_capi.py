@@ -11,7 +11,9 @@ from __future__ import annotations
 
 import ctypes
 import os
+import sys
 import threading
+import warnings
 
 import torch  # noqa: F401  (must precede the library load, see module docstring)
 
@@ -81,11 +83,13 @@ _lock = threading.Lock()
 
 # Host fast paths over the same library (csrc/native.cpp, built beside it).  Each
 # returns None for whatever it does not take; without the module the Python
-# forms serve every call.
+# forms serve every call, a step of short requests then at half the speed.
 try:
     from . import _native as native
-except ImportError:
+except ImportError as e:
     native = None
+    warnings.warn(f"the native module of the host calls is not loaded ({e}); build it for this interpreter with "
+                  f"`make -C dllm-serve_amd/csrc PYTHON={sys.executable}`", RuntimeWarning, stacklevel=2)
 
 
 def load(path: str | None = None) -> ctypes.CDLL:

@@ -4,6 +4,9 @@ rejects invalid requests before touching the GPU (no kernel is launched)."""
 import ctypes
 import os
 import re
+import shutil
+import subprocess
+import sys
 
 import pytest
 
@@ -236,3 +239,26 @@ def test_launch_shape_queries():
     assert _capi.block_cached_launch_shape(2, 32, 4128, 32, 32, 128)["n_split"] > 1
     with pytest.raises(RuntimeError):
         _capi.varlen_launch_shape(1, 8, 8, 32, 32, 64)
+
+
+PKG = os.path.dirname(os.path.abspath(_capi.__file__))
+CSRC = os.path.join(os.path.dirname(PKG), "csrc")
+
+
+def _python(code, path):
+    return subprocess.run([sys.executable, "-W", "always", "-c", code], env=dict(os.environ, PYTHONPATH=str(path)),
+                          capture_output=True, text=True, timeout=300)
+
+
+@pytest.mark.parametrize("broken", ["absent", "not a library"])
+def test_native_module_that_does_not_load_is_reported(tmp_path, broken):
+    """A step costs twice as much without the native module: that is said."""
+    shutil.copytree(PKG, tmp_path / "dllm_serve_amd", ignore=shutil.ignore_patterns("__pycache__"))
+    so = tmp_path / "dllm_serve_amd" / "_native.so"
+    so.unlink()
+    if broken != "absent":
+        so.write_bytes(b"nothing that the loader takes")
+    r = _python("from dllm_serve_amd import _capi; assert _capi.native is None; _capi.load()", tmp_path)
+    assert r.returncode == 0, r.stderr
+    assert "RuntimeWarning" in r.stderr and "native module" in r.stderr
+    assert "RuntimeWarning" not in _python("from dllm_serve_amd import _capi; assert _capi.native", os.path.dirname(PKG)).stderr

@@ -262,3 +262,14 @@ def test_native_module_that_does_not_load_is_reported(tmp_path, broken):
     assert r.returncode == 0, r.stderr
     assert "RuntimeWarning" in r.stderr and "native module" in r.stderr
     assert "RuntimeWarning" not in _python("from dllm_serve_amd import _capi; assert _capi.native", os.path.dirname(PKG)).stderr
+
+
+def test_library_builds_without_torch():
+    """The C ABI needs no torch; the native module is built for the interpreter that is named."""
+    def commands(python):
+        return subprocess.run(["make", "-n", "-B", "-C", CSRC, f"PYTHON={python}"], check=True, capture_output=True,
+                              text=True).stdout
+
+    bare = commands(f"{sys.executable} -S")  # -S: no site-packages, no torch
+    assert "libdllm_attn.so" in bare and "native.cpp" not in bare
+    assert "native.cpp" in commands(sys.executable)

@@ -273,3 +273,12 @@ def test_library_builds_without_torch():
     bare = commands(f"{sys.executable} -S")  # -S: no site-packages, no torch
     assert "libdllm_attn.so" in bare and "native.cpp" not in bare
     assert "native.cpp" in commands(sys.executable)
+
+
+def test_build_names_its_own_interpreter(monkeypatch):
+    import __graft_entry__ as entry
+
+    seen = []
+    monkeypatch.setattr(entry.subprocess, "run", lambda cmd, **kw: seen.append(cmd))
+    entry.build()
+    assert f"PYTHON={sys.executable}" in seen[0]

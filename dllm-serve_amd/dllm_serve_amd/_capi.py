@@ -93,8 +93,9 @@ except ImportError as e:
 
 
 def load(path: str | None = None) -> ctypes.CDLL:
-    """Load (once) and return the library; raise RuntimeError if it is absent."""
-    global _lib
+    """Load (once) and return the library; raise RuntimeError if it is absent.
+    With a `path` other than the package's own, every call goes to that library."""
+    global _lib, native
     with _lock:
         if _lib is not None:
             return _lib
@@ -104,6 +105,8 @@ def load(path: str | None = None) -> ctypes.CDLL:
                 f"{LIB_NAME} not found at {p}; build it with `make -C dllm-serve_amd/csrc` "
                 "(or __graft_entry__.build()). There is no CPU fallback for this path."
             )
+        if os.path.realpath(p) != os.path.realpath(LIB_PATH):
+            native = None  # it is linked to the library beside it, not to this one
         lib = ctypes.CDLL(p)
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(lib, name)

@@ -282,3 +282,14 @@ def test_build_names_its_own_interpreter(monkeypatch):
     monkeypatch.setattr(entry.subprocess, "run", lambda cmd, **kw: seen.append(cmd))
     entry.build()
     assert f"PYTHON={sys.executable}" in seen[0]
+
+
+def test_another_library_serves_every_call(tmp_path):
+    """load(path): the native module, which is linked to the package's own library, steps back."""
+    shutil.copy(_capi.LIB_PATH, tmp_path / "other.so")
+    r = _python(f"from dllm_serve_amd import _capi; assert _capi.native; _capi.load({str(tmp_path / 'other.so')!r}); "
+                "assert _capi.native is None", os.path.dirname(PKG))
+    assert r.returncode == 0, r.stderr
+    r = _python("from dllm_serve_amd import _capi; _capi.load(_capi.LIB_PATH); assert _capi.native",
+                os.path.dirname(PKG))
+    assert r.returncode == 0, r.stderr

@@ -313,3 +313,27 @@ def test_softmax_max_sample_overflow(dev):
     x0, p = _run_k8_sample(t.to(dev), [1.0, 1.0], 7, 0)
     assert x0[0] == 41 and np.isnan(torch.from_numpy(p[:1].view(np.int16)).view(torch.bfloat16).float().item())
     _check_sample(bits(t[1:]), np.array([1.0]), 7, 1, x0[1:], p[1:])
+
+
+@pytest.mark.parametrize("V", [64, 4104, 33288])
+@pytest.mark.parametrize("workspace", [False, True])
+def test_softmax_max_sample_without_a_threshold(dev, V, workspace):
+    """Rows whose values stay below the gap are computed whole; one large value
+    anywhere (first and last column, a later round of chunks) ends that."""
+    print(f"softmax_max_sample no threshold V={V} workspace={workspace}", flush=True)
+    g = torch.Generator().manual_seed(V)
+    at = [None, 0, 7, V // 2, V - 9, V - 1]
+    M, T = len(at), 0.4
+    t = (torch.randn(M, V, generator=g) - 6.0).to(torch.bfloat16)
+    for r, c in enumerate(at):
+        if c is not None:
+            t[r, c] = 12.0
+    logits = t.to(dev)
+    temps = torch.full((M,), T, dtype=torch.float64, device=dev)
+    x0 = torch.full((M,), -1, dtype=torch.int64, device=dev)
+    p = torch.zeros(M, dtype=torch.bfloat16, device=dev)
+    need = _capi.softmax_max_split_workspace_size(M, V)
+    ws = torch.empty(need, dtype=torch.uint8, device=dev) if workspace and need else None
+    _capi.softmax_max_sample(logits, temps, 17, 0, x0, p, ws)
+    assert all(int(x0[r]) == c for r, c in enumerate(at) if c is not None)
+    _check_sample(bits(t), np.full(M, T), 17, 0, x0.cpu().numpy(), bits(p))

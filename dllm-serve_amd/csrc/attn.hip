@@ -1451,23 +1451,27 @@ static int common_checks(const char* name, const void* q, const void* k, const v
   return DLLM_OK;
 }
 
-// Raise a kernel's dynamic-LDS limit (once per kernel and device).
+// Raise a kernel's dynamic-LDS limit (once per kernel and device; a thread
+// remembers the devices of each kernel of a type as bits).
 template <typename KernelFn>
 static int set_lds(KernelFn fn, int bytes, const char* name) {
-  static thread_local const void* done[16];
-  static thread_local int done_dev[16];
+  constexpr int kKernels = 24;  // of one type: the block-cached form has twelve
+  static thread_local const void* done[kKernels];
+  static thread_local uint64_t done_dev[kKernels];
   static thread_local int n_done = 0;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) dev = -1;
+  const uint64_t bit = dev >= 0 && dev < 64 ? 1ull << dev : 0;
   const void* key = reinterpret_cast<const void*>(fn);
-  for (int i = 0; i < n_done; ++i)
-    if (done[i] == key && done_dev[i] == dev) return DLLM_OK;
+  int i = 0;
+  while (i < n_done && done[i] != key) ++i;
+  if (i < n_done && (done_dev[i] & bit)) return DLLM_OK;
   hipError_t e = hipFuncSetAttribute(key, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   if (e != hipSuccess) return fail(DLLM_ERR_HIP, "%s: hipFuncSetAttribute(LDS %d B): %s", name, bytes, hipGetErrorString(e));
-  if (n_done < 16) {
-    done[n_done] = key;
-    done_dev[n_done] = dev;
-    ++n_done;
+  if (i < kKernels) {
+    done[i] = key;
+    done_dev[i] |= bit;
+    if (i == n_done) ++n_done;
   }
   return DLLM_OK;
 }

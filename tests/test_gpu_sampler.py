@@ -118,11 +118,15 @@ def test_softmax_max_ties_and_neg_inf(dev):
 def _unmask_case(rng, n_seq, max_win, tie_levels):
     tokens, params, rows = [], [], 0
     for b in range(n_seq):
-        n = int(rng.integers(0, max_win + 1))
+        n = int(rng.integers(0, max_win + 1)) if b else max_win
         pad = int(rng.integers(0, 9))
         tok = rng.integers(0, 1000, n + pad)
         tok[pad:][rng.random(n) < rng.random()] = MASK
-        params.append((len(tokens) + pad, n, rows, int(rng.integers(-1, 9)), int(rng.random() < 0.5)))
+        steps = int(rng.integers(-1, 9))
+        if b == 0:  # the longest window, masked to its last position, of which some are unmasked
+            tok[-1] = MASK
+            steps = 2
+        params.append((len(tokens) + pad, n, rows, steps, int(rng.random() < 0.5)))
         tokens.extend(tok.tolist())
         rows += n
     conf = f32_to_bf16_bits(np.round(rng.random(rows) * tie_levels) / tie_levels) if tie_levels else \
@@ -132,19 +136,22 @@ def _unmask_case(rng, n_seq, max_win, tie_levels):
 
 
 @pytest.mark.parametrize("n_seq,max_win,ties", [(64, 300, 0), (64, 300, 16), (8, 8192, 64), (3, 1, 0), (32, 64, 2),
+                                               # edges of the one-wavefront forms (64, 256 and 1024 positions)
                                                (20, 65, 4), (20, 256, 0), (20, 257, 3), (20, 1024, 8),
-                                               (20, 1025, 8)])  # edges of the one-wavefront forms
+                                               (20, 1025, 8)])
 def test_unmask_matches_oracle(dev, n_seq, max_win, ties):
     print(f"unmask n_seq={n_seq} max_win={max_win} ties={ties}", flush=True)
     rng = np.random.default_rng(n_seq * 31 + max_win + ties)
     tokens, params, conf, x0 = _unmask_case(rng, n_seq, max_win, ties)
+    assert max(w[1] for w in params) == max_win  # the kernel form goes by the longest window
     want, want_n = osm.unmask_step(tokens, params, x0, conf, MASK)
+    assert want_n[0] > 0
     t = torch.from_numpy(tokens).to(dev)
     p = torch.tensor(params, dtype=torch.int32).to(dev)
     cf = torch.from_numpy(conf.view(np.int16)).view(torch.bfloat16).to(dev)
     xd = torch.from_numpy(x0).to(dev)
     nun = torch.full((n_seq,), -1, dtype=torch.int32, device=dev)
-    _capi.lowconf_unmask(t, p, n_seq, max(w[1] for w in params), xd, cf, MASK, nun)
+    _capi.lowconf_unmask(t, p, n_seq, max_win, xd, cf, MASK, nun)
     torch.cuda.synchronize()
     got = t.cpu().numpy()
     assert np.array_equal(nun.cpu().numpy(), want_n)

@@ -48,7 +48,7 @@ def test_c1_single_layer(dev):
     ([1000], 4, 4),
     ([300, 384, 1, 257, 383], 32, 32),               # 257..384 M rows, 160 pairs: one 12-wavefront workgroup each
     ([64, 96, 7, 90] * 10, 16, 4),                     # the same launch with GQA (96 x 4 = 384 M rows, 160 pairs)
-    ([300, 384, 1, 257, 383], 16, 16),               # the same rows, 80 pairs: three 4-wavefront workgroups each
+    ([300, 384, 1, 257, 383], 16, 16),               # the same rows, 80 pairs: three piped workgroups of four wavefronts each
     ([500, 33, 1], 32, 1),                             # MQA, g = 32: one KV row serves 32 M rows
     ([260, 7], 64, 1),                                 # g = 64
 ])
@@ -148,7 +148,8 @@ def test_varlen_strided_views(dev):
 
 
 @pytest.mark.parametrize("lens,Hq,Hkv,pad", [
-    ([150, 260, 1], 8, 2, 8),               # 4-wavefront launch
+    ([150, 260, 1], 8, 2, 8),               # piped launch, one wavefront
+    ([150, 260, 1] * 8, 16, 4, 8),          # plain 4-wavefront launch (864 blocks)
     ([300, 384, 1, 257, 383] * 2, 16, 16, 24),  # 160 pairs of 257..384 M rows: 12-wavefront launch
     ([2100, 40], 4, 4, 8),                  # key streams >= 2048: 8-wavefront launch
 ])
@@ -302,16 +303,22 @@ def test_block_cached_without_a_cache(dev, prefix, Hq, Hkv):
     assert_attn_close(o, ref, "blocks only")
 
 
-@pytest.mark.parametrize("lens,Hq,Hkv", [
-    ([333, 20, 517], 28, 4),     # 4-wavefront launch: 29 m-tiles, chunks of 16, 348 blocks in a grid of 384
-    ([300] * 5, 32, 32),         # 12-wavefront launch: 160 pairs, chunks of 1, grid 160
-    ([2500, 100], 8, 2),         # 8-wavefront launch: 40 m-tiles, chunks of 16, 160 blocks in a grid of 256
-    ([129, 5, 131], 8, 8),       # 4-wavefront launch: 2 m-tiles, chunks of 2, 48 blocks in a grid of 48
+@pytest.mark.parametrize("lens,Hq,Hkv,wavefronts,blocks,grid", [
+    ([333, 20, 517], 28, 4, 4, 348, 384),              # piped: 29 m-tiles of 128 rows, chunks of 16
+    ([129, 5, 131], 8, 8, 1, 120, 120),                # piped, one wavefront: 5 m-tiles of 32 rows, chunks of 5
+    ([333, 20, 517, 400, 290], 28, 4, 4, 580, 640),    # plain: over 384 blocks, 29 m-tiles, chunks of 16
+    ([129, 5, 131] * 11, 8, 8, 4, 528, 528),           # plain: 2 m-tiles, chunks of 2
+    ([300] * 5, 32, 32, 12, 160, 160),                 # 160 pairs, chunks of 1
+    ([2500, 100], 8, 2, 8, 160, 256),                  # 40 m-tiles of 256 rows, chunks of 16
 ])
-def test_varlen_xcd_interleave_covers_every_block(dev, lens, Hq, Hkv):
+def test_varlen_xcd_interleave_covers_every_block(dev, lens, Hq, Hkv, wavefronts, blocks, grid):
     """Logical blocks are dealt to the XCDs in chunks and the grid is padded
     to a multiple of 8 chunks: every output row is written (none left at the
     NaN fill) and matches the oracle."""
+    shape = _capi.varlen_launch_shape(len(lens), max(lens), max(lens), Hq, Hkv, 128)
+    assert shape["wavefronts"] == wavefronts and shape["grid"] == grid
+    # (four wavefronts: the piped form up to 384 blocks)
+    assert len(lens) * Hkv * -(-max(lens) * Hq // Hkv // (32 * wavefronts)) == blocks
     print(f"varlen xcd interleave lens={lens} Hq={Hq} Hkv={Hkv}", flush=True)
     q, k, v, cu = configs.packed_qkv(lens, Hq, Hkv, 128, seed=7 + sum(lens))
     o = _run_varlen(q, k, v, cu, dev, o_init=torch.full(q.shape, float("nan"), dtype=torch.bfloat16))
@@ -463,11 +470,18 @@ def test_block_cached_d_parts_equal_a_batch(dev, paged, n_seg, Hq, Hkv, lq, nc, 
         torch.cuda.synchronize()
         return o
 
+    # the grid of `parts` workgroups per (segment, KV head, row block), padded to eight chunks of a pair's
+    mblocks = -(-(lq * Hq // Hkv) // 32)
+
+    def grid(n, d_parts):
+        grain = 8 * min(16, d_parts * mblocks)
+        return -(-n * Hkv * mblocks * d_parts // grain) * grain
+
     shape = _capi.block_cached_launch_shape(n_seg, lq, nc + lq, Hq, Hkv, D)
-    blocks = n_seg * Hkv * -(-(lq * Hq // Hkv) // 32)
-    assert shape["n_split"] == 1 and shape["row_blocks"] == 1 and shape["grid"] >= parts * blocks
+    assert shape == dict(row_blocks=1, n_split=1, grid=grid(n_seg, parts))
+    assert all(grid(n_seg, p) != shape["grid"] for p in (1, 2, 4) if p != parts)
     full = _capi.block_cached_launch_shape(n_seg * copies, lq, nc + lq, Hq, Hkv, D)
-    assert full["n_split"] == 1 and full["grid"] < 2 * copies * blocks + 128
+    assert full["n_split"] == 1 and (full["row_blocks"] == 2 or full["grid"] == grid(n_seg * copies, 1))
     alone, batch = run(1), run(copies)
     for i in (0, copies - 1):
         part = batch[i * n_seg * lq:(i + 1) * n_seg * lq]

@@ -821,10 +821,12 @@ constexpr int CK_STAGE = 2 * CK_TILE * 256;
 // ([4 tiles][4 RB wavefronts][64] words); the final merge reuses both
 constexpr int ck_lds_bytes(int rb) { return 2 * CK_STAGE + 4 * 4 * rb * 64 * 4; }
 
-// Cache and block rows of a segment are read by exactly one workgroup, each
-// 16-byte piece by one lane of one DMA instruction: streaming loads (the q
-// loads keep the default policy: a lane reads each q line in four 32-byte
-// steps and relies on the cache between them).
+// Streaming loads: a 16-byte piece of a cache or block row is read by one lane
+// of one DMA instruction of a workgroup.  The workgroups that read the same rows
+// (row blocks and head-dim parts of one segment and KV head) do so at about the
+// same time and through one L2.  Without the hint every shape was 1-10 % slower,
+// caches from HBM.  (The q loads keep the default policy: a lane reads each q
+// line in four 32-byte steps and relies on the cache between them.)
 __device__ __forceinline__ void gdma16(const void* g, uint8_t* lds_dst) {
   __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)lds_dst, 16, 0, kStreamAux);
 }
@@ -1507,9 +1509,12 @@ static DensePlan dense_plan(int n_seg, int max_seqlen_q, int max_seqlen_k, int H
   // 32 heads, in us, 4 wavefronts plain / piped with 4, 2, 1: 1 x 256 tokens
   // 9.1 / 9.0, 8.2, 8.0; 1 x 512 13.7 / 13.0, 11.8, 12.7; 1 x 640 16.2 / 15.3,
   // 19.3, 16.3; 4 x 256 10.5 / 10.2, 12.4, 11.6.  Four wavefronts up to three
-  // workgroups on two CUs: 1 x 1280 (320 workgroups) 40.0 / 38.5, 4 x 384 (384)
-  // 19.6 / 19.4, 8 x 384 as 768 29 / 30 (not taken); and from 192 keys on: 4 x
-  // 139 tokens 7.8 / 7.9, 6 x 139 10.95 / 11.1, 4 x 200 9.4 / 9.15.
+  // workgroups on two CUs.  There the two forms are close, medians of three
+  // alternating runs: 1 x 1280 (320 workgroups) 40.1 / 38.9, 1 x 1500 (384) 48.1 /
+  // 47.0, 2 x 700 26.9 / 26.7, 4 x 384 19.3 / 19.2, 6 x 200 14.15 / 14.05, but 5 x
+  // 256 15.1 / 15.3; 8 x 384 as 768 29 / 30 (not taken).  Below 192 keys neither
+  // wins: 4 x 139 tokens 8.7 / 8.9, 6 x 139 11.8 / 12.1, 6 x 128 8.9 / 8.65; the
+  // plain form is kept there.
   if (!wide) {
     const int64_t pairs = (int64_t)n_seg * Hkv;
     auto groups = [&](int nw) { return pairs * ((m_rows + 32 * nw - 1) / (32 * nw)); };

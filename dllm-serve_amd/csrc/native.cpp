@@ -4,8 +4,9 @@
 // A denoising step of one short request is bound by the host: per layer the
 // Python form of Attention.forward and RotaryEmbedding.forward spent 11 and 14
 // us (attribute reads, views, 20-odd ctypes conversions) on launches whose
-// kernels take 9 and 3 us; these forms take 7 and 5 (the step of one 384-token
-// request over 32 layers: 1027 -> 597 us, then bound by the kernels).  Every function here takes the ordinary case only
+// kernels take 9 and 3 us; these forms take 7 and 5.  The step of one 384-token
+// request over 32 layers, whose kernels sum to about 400 us: 1047 -> 522 us, which
+// still varies with the host.  Every function here takes the ordinary case only
 // and returns None for anything else -- another type, layout, device or tensor
 // class, and what the C ABI refuses before it launches anything -- and the Python
 // form, which raises what is to be raised, runs then.  A failure of the HIP

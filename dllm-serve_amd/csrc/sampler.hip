@@ -495,7 +495,7 @@ __global__ __launch_bounds__(256) void smx_merge_kernel(SmxArgs a) {
   smx_finish(a, row, m, s, idx);
 }
 
-// Workgroups per row.  A CU takes in at most ~26 GB a millisecond, ~10 us for a
+// Workgroups per row.  A CU takes in at most ~26 KB a microsecond, ~10 us for a
 // row of 253 KB, so few rows are spread over several CUs; the second launch
 // (~2.5 us) pays for that up to 64 rows, and with noise, whose integer hash
 // keeps a CU busy for 35 us a row, wherever CUs would stay idle.  Measured at
@@ -596,7 +596,8 @@ __global__ __launch_bounds__(256) void lowconf_unmask_kernel(UnmaskArgs a) {
 // chain of latencies (parameters, tokens and confidences, x0); the bitwise
 // search's 32 counts were the longest part of it as workgroup sums (two
 // barriers each), and are ballots and scalar bit counts here, with x0 loaded
-// beside the confidences.  8 windows of 32 positions on an MI355X: 11.2 -> 3.3 us.
+// beside the confidences.  8 windows of 32 positions on an MI355X: 11.2 -> 3.3 us
+// in a loop of this launch alone, 11.5 -> 3.9 traced inside a sampling step.
 template <int KPL>
 __global__ __launch_bounds__(64) void lowconf_unmask_wave_kernel(UnmaskArgs a) {
   const int b = blockIdx.x;

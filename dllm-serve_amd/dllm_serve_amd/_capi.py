@@ -221,7 +221,7 @@ def varlen_launch_shape(n_seg, max_seqlen_q, max_seqlen_k, Hq, Hkv, D) -> dict:
 
 def block_cached_launch_shape(n_seg, max_q, max_keys, Hq, Hkv, D) -> dict:
     """Launch shape K3b picks for these sizes (no launch): row blocks per
-    workgroup, key splits, grid."""
+    workgroup, workgroups along the keys (`n_split`), grid."""
     vals = [ctypes.c_int(0) for _ in range(3)]
     _check(load().dllm_attn_block_cached_launch_shape(n_seg, max_q, max_keys, Hq, Hkv, D,
                                                       *[ctypes.byref(x) for x in vals]),

@@ -5,9 +5,10 @@
  * caller's current stream, e.g. torch.cuda.current_stream().cuda_stream),
  * takes raw device pointers, element strides and sizes, never allocates
  * device memory and never throws.  Return value 0 means the work was
- * enqueued; a negative DLLM_ERR_* code means nothing was launched and
- * dllm_last_error() describes why (thread-local, valid until the next call
- * on the same thread).
+ * enqueued; a negative DLLM_ERR_* code is described by dllm_last_error()
+ * (thread-local, valid until the next call on the same thread).  Nothing was
+ * launched then, except perhaps with DLLM_ERR_HIP: the runtime reports an
+ * error, of this call or one still pending, after a launch.
  *
  * Tensors are bfloat16 (raw 16-bit patterns, type dllm_bf16), row-major,
  * innermost dimension contiguous.  "Rows" are tokens: q is [rows, Hq, D],
@@ -129,8 +130,8 @@ int dllm_attn_varlen_launch_shape(int n_seg, int max_seqlen_q, int max_seqlen_k,
  */
 size_t dllm_attn_block_cached_workspace_size(int n_seg, int max_q, int max_keys, int Hq, int Hkv, int D);
 /* Launch shape of dllm_attn_block_cached_fwd for these sizes, without
- * launching: 32-row blocks per workgroup (1 or 2), key splits (> 1 adds the
- * combine launch) and the grid.  No counterpart in the reference; for tests
+ * launching: 32-row blocks per workgroup (1 or 2), workgroups along the keys
+ * (> 1 adds the combine launch) and the grid.  No counterpart in the reference; for tests
  * and profiles.  Any output pointer may be null. */
 int dllm_attn_block_cached_launch_shape(int n_seg, int max_q, int max_keys, int Hq, int Hkv, int D,
                                         int* row_blocks, int* n_split, int* grid);
